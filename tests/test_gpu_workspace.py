@@ -1,0 +1,40 @@
+"""lkhip_matmul's kept workspaces: products that share them equal the same
+products alone."""
+import numpy as np
+import pytest
+
+from lokal_amd import kernels as K
+from lokal_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def test_matmul_workspace_is_shared_in_stream_order():
+    """Products of several sizes, back to back on the null stream and on two
+    created streams, use kept workspaces: each equals the same product alone,
+    also after a stream and every weight are gone."""
+    rng = np.random.default_rng(5)
+    shapes = [(2048, 2048, 100), (4864, 896, 64), (1024, 4864, 200), (6000, 896, 512)]
+    for _ in range(2):
+        ws, xs, alone = [], [], []
+        for rows, cols, n in shapes:
+            ws.append(K.Weight(synth.Q8_0, rows, cols, synth.gen_weight(synth.Q8_0, 3, f"{rows}", rows, cols).data))
+            xs.append(K.DeviceArray.from_numpy(rng.standard_normal((n, cols)).astype(np.float32)))
+            y = K.DeviceArray((n, rows))
+            K.matmul(ws[-1], xs[-1], n, y)
+            alone.append(y.numpy())
+        streams = [K.Stream(), K.Stream()]
+        outs = []
+        for rep in range(3):
+            for st in (None, *streams):
+                for w, x, (rows, cols, n) in zip(ws, xs, shapes):
+                    y = K.DeviceArray((n, rows))
+                    K.matmul(w, x, n, y, stream=st.ptr if st else None)
+                    outs.append(y)
+        K.synchronize()
+        for i, y in enumerate(outs):
+            assert np.array_equal(y.numpy(), alone[i % len(shapes)]), i
+        for st in streams:
+            st.close()
+        for w in ws:
+            w.close()
