@@ -189,7 +189,7 @@ static int weight_create(uint32_t type, size_t rows, size_t cols, const void* ho
     return LKHIP_OK;
 }
 
-// lkhip_matmul's workspaces (split-K partials), kept per stream: calls
+// lkhip_matmul's workspaces (X planes, split-K partials), kept per stream: calls
 // on one stream run in order, so they share one buffer, and a call holds the
 // lock until its launches are enqueued, so another thread's cannot come between.
 // hipMallocAsync + hipFreeAsync cost 13 us per call, more than a small product.
@@ -613,7 +613,7 @@ enum HeadMode { HEAD_NONE = 0, HEAD_LAST = 1, HEAD_ALL = 2 };
 struct Rows {
     uint32_t cap = 0;
     DevBuf meta;   // u32 [ids | pos | slots | ctx | steps], cap each
-    DevBuf x, xn, qkv, att, inner, logits, gpart, apart, out_ids, keys;
+    DevBuf x, xn, qkv, att, inner, logits, gpart, apart, out_ids, keys, planes;
     size_t out_ids_cap = 0;
     uint32_t* h_meta = nullptr;  // pinned, 5 * cap
     ~Rows() {
@@ -1291,6 +1291,7 @@ static int rows_alloc(const lkhip_engine* e, Rows& R, uint32_t cap, uint32_t max
         (rc = dev_alloc(R.logits, lrows * c.vocab_size * 4)) ||
         (rc = dev_alloc(R.keys, lrows * ((c.vocab_size + LK_ARGMAX_SLICE - 1) / LK_ARGMAX_SLICE) * 8)) ||
         (rc = dev_alloc(R.gpart, rows_gemm_part(e, cap) * 4)) ||
+        (rc = dev_alloc(R.planes, lk_planes_bytes(cap, std::max(std::max(h, I), (size_t)e->qd)))) ||
         (rc = dev_alloc(R.apart, lk_attn_scratch_floats(cap, c.num_attention_heads, max_seq, (size_t)cap * c.num_key_value_heads) * 4)))
         return rc;
     HIP_OR_FAIL(hipHostMalloc((void**)&R.h_meta, 5 * (size_t)cap * 4, hipHostMallocDefault));
@@ -1299,6 +1300,7 @@ static int rows_alloc(const lkhip_engine* e, Rows& R, uint32_t cap, uint32_t max
 
 static hipError_t rows_gemm(Rows& R, LkGemmArgs a, int mode, hipStream_t st) {
     a.part = R.gpart.as<float>();
+    a.planes = R.planes.p;
     a.ks = 0;  // the planned split
     return lk_gemm_launch(a, mode, st);
 }
@@ -1366,6 +1368,7 @@ static hipError_t enqueue_rows(const lkhip_engine* e, Rows& R, uint32_t n, const
             a.ldx = h;
             a.ldy = qkvd;
             a.part = part;
+            a.planes = R.planes.p;
             if (!qkv_mixed(ly)) {
                 RSTEP(lk_gemm_launch(a, LK_MV_STORE, st, &ks));
             } else {
@@ -1435,6 +1438,7 @@ static hipError_t enqueue_rows(const lkhip_engine* e, Rows& R, uint32_t n, const
             a.ldx = qd;
             a.ldy = h;
             a.part = part;
+            a.planes = R.planes.p;
             RSTEP(lk_gemm_launch(a, LK_MV_ACC, st, &ks));
         }
         RSTEP(lk_rows_accnorm_launch(x, part, ks, n, h, ly.post_norm.as<float>(), c.rms_norm_eps, xn, st));
@@ -1462,6 +1466,7 @@ static hipError_t enqueue_rows(const lkhip_engine* e, Rows& R, uint32_t n, const
             a.ldx = I;
             a.ldy = h;
             a.part = part;
+            a.planes = R.planes.p;
             RSTEP(lk_gemm_launch(a, LK_MV_ACC, st, &pend));
         }
     }
@@ -2396,7 +2401,7 @@ extern "C" int lkhip_matmul(const lkhip_weight* w, const float* x, size_t n_rows
     const int mode = accumulate ? LK_MV_ACC : LK_MV_STORE;
     const LkGemmPlan p = lk_gemm_plan(d.type, d.rows, d.cols, (uint32_t)n_rows, mode);
     hipStream_t st = (hipStream_t)stream;
-    const size_t bytes = p.part_floats * 4;
+    const size_t part_bytes = (p.part_floats * 4 + 255) / 256 * 256, bytes = part_bytes + p.plane_bytes;
     std::unique_lock<std::mutex> lk(g_ws_mu, std::defer_lock);
     if (bytes) lk.lock();
     void* const kept = bytes ? ws_get(st, bytes) : nullptr;
@@ -2414,8 +2419,9 @@ extern "C" int lkhip_matmul(const lkhip_weight* w, const float* x, size_t n_rows
     a.x = x;
     a.ldx = (uint32_t)ldx;
     a.ldy = (uint32_t)ldy;
-    a.part = (float*)part;
-    a.ks = p.ks;
+    a.part = p.part_floats ? (float*)part : nullptr;
+    a.planes = p.plane_bytes ? (uint8_t*)part + part_bytes : nullptr;
+    a.ks = p.tile.kind ? p.tile.ks : p.ks;
     hipError_t e = lk_gemm_launch(a, mode, st);
     if (bytes && !kept) (void)hipFreeAsync(part, st);
     if (e != hipSuccess) return fail(LKHIP_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));

@@ -35,25 +35,6 @@
 
 namespace lkg {
 
-// Epilogue of one output element: segment n (global index over segments).
-__device__ __forceinline__ void emit(const LkGemmArgs& a, int mode, uint32_t b, uint32_t n, float v, float u) {
-    if (mode == LK_MV_SWIGLU) {
-        a.seg[0].out[(size_t)b * a.ldy + n] = silu_mul(v, u);
-        return;
-    }
-    uint32_t si = 0, nb = 0;
-    while (si + 1 < a.nseg && n >= nb + a.seg[si].w.rows) {
-        nb += a.seg[si].w.rows;
-        si++;
-    }
-    const LkSeg& s = a.seg[si];
-    const uint32_t nl = n - nb;
-    if (s.bias) v += s.bias[nl];
-    float* o = s.out + (size_t)b * a.ldy + nl;
-    if (mode == LK_MV_ACC) *o += v;
-    else *o = v;
-}
-
 template <int WT, int MB, int MODE>
 __global__ __launch_bounds__(256) void gemm_kernel(const LkGemmArgs a) {
     constexpr bool SW = MODE == LK_MV_SWIGLU;
@@ -823,8 +804,56 @@ static uint32_t gemm_mb(uint32_t n_rows) { return n_rows <= 16 ? 1 : 2; }
 #define LK_GEMM_WIDE_N 16384u
 #endif
 
+// gemm_tile.hip from 33 rows on, where the product is large enough to pay for
+// its X conversion launch (2.5-8 us): from 200,000 sums.  Both sides measured
+// (us on the device, the kernels that read X themselves / the tile kernels,
+// conversion and K-split sums included): Q8_0 4864 x 896 at 64 / 512 rows
+// 17.3 / 11.8 and 47.6 / 25.4, 896 x 4864 at 64 / 512 rows 17.4 / 20.2 and
+// 48.6 / 32.8, 1152 x 896 at 64 rows 9.3 / 10.7, 4035 x 4032 at 50 rows 28.9 /
+// 24.9, 151936 x 896 at 64 rows 105.5 / 53.2; F16 576 x 1536 at 256 rows 13.7
+// / 17.1, 1536 x 576 15.0 / 10.1; Q4_K 2048 x 5632 at 256 rows 78.7 / 38.9.
+#define LK_TILE_MIN_ROWS 33u
+#define LK_TILE_MIN_SUMS 200000u
+static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_rows, int mode) {
+    LkTilePlan p{};
+    const bool sw = mode == LK_MV_SWIGLU;
+    if (n_rows < LK_TILE_MIN_ROWS || (uint64_t)N * (sw ? 2 : 1) * n_rows < LK_TILE_MIN_SUMS) return p;
+    if (!lkg::gemm16_on(type) || (type == LK_Q8_0 && K % 64)) return p;  // whole 64-column stages of block scales
+    // 32-bit offsets inside a block's rows and the planes
+    if (lk_planes_bytes(n_rows, K) >> 32 || (uint64_t)K * 64 >> 31) return p;
+    const uint32_t nck = (K + lkg::KC - 1) / lkg::KC;
+    auto blocks = [&](uint32_t bn, uint32_t bm) { return ((N + bn - 1) / bn) * ((n_rows + bm - 1) / bm); };
+    // The largest tile that leaves every CU several waves: a lone wave per SIMD
+    // issues a vector instruction every 7 cycles, three or four together one
+    // every 3.5-4, and a stage is bound by that.  Few tiles: the small one, K
+    // split over the grid when even that leaves CUs without a block; a deep K
+    // amortises 8-wave blocks that share X, with K split over 256 of them.
+    // Q8_0 4864 x 896, 512 rows, by kind (kernel us): small 22.9, mid 19.1, large
+    // 21.3, split (8) 31.8; 896 x 896: 9.2 / 11.5 / 14.5 / 9.7; 896 x 4864:
+    // 32.1 / 47.4 / 60.1 / 20.0; 151936 x 896, 64 rows: 72 / 55 / 47 / 110.
+    uint32_t ks = 1;
+    if (sw) {
+        p.kind = blocks(64, 64) >= 256 ? LK_TILE_LARGE : LK_TILE_SMALL;
+        if (p.kind == LK_TILE_SMALL) ks = 192 / blocks(64, 32);
+    } else if (blocks(128, 64) >= 1024) {
+        p.kind = LK_TILE_LARGE;
+    } else if (blocks(64, 64) >= 512) {
+        p.kind = LK_TILE_MID;
+    } else if (K <= 1024) {
+        p.kind = LK_TILE_SMALL;
+        ks = 192 / blocks(64, 32);
+    } else {
+        p.kind = LK_TILE_SPLIT;
+        ks = (256 + blocks(256, 64) - 1) / blocks(256, 64);
+    }
+    if (ks > nck) ks = nck;
+    if (ks < 1) ks = 1;
+    const uint32_t per = (nck + ks - 1) / ks;
+    p.ks = (nck + per - 1) / per;
+    return p;
+}
+
 LkGemmPlan lk_gemm_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_rows, int mode) {
-    (void)type;
     LkGemmPlan p{};
     p.mb = gemm_mb(n_rows);
     const uint32_t gx = (N + 63) / 64, gy = (n_rows + 16 * p.mb - 1) / (16 * p.mb);
@@ -835,7 +864,10 @@ LkGemmPlan lk_gemm_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_rows, 
     if (ks < 1) ks = 1;
     const uint32_t per = (nck + ks - 1) / ks;
     p.ks = (nck + per - 1) / per;
-    p.part_floats = p.ks > 1 ? (size_t)p.ks * n_rows * N * (mode == LK_MV_SWIGLU ? 2 : 1) : 0;
+    p.tile = tile_plan(type, N, K, n_rows, mode);
+    if (p.tile.kind) p.plane_bytes = lk_planes_bytes(n_rows, K);
+    const uint32_t most = p.ks > p.tile.ks ? p.ks : p.tile.ks;
+    p.part_floats = most > 1 ? (size_t)most * n_rows * N * (mode == LK_MV_SWIGLU ? 2 : 1) : 0;
     return p;
 }
 
@@ -857,6 +889,20 @@ hipError_t lk_gemm_launch(LkGemmArgs a, int mode, hipStream_t st, uint32_t* defe
         for (uint32_t i = 0; i + 1 < a.nseg; i++)
             if (a.seg[i].w.rows % 16) return hipErrorInvalidValue;
     if (a.ldx % 4 || (size_t)(uintptr_t)a.x % 16) return hipErrorInvalidValue;  // float4 X loads
+    const LkGemmPlan p = lk_gemm_plan(type, a.N, a.K, a.n_rows, mode);
+    hipError_t e;
+    if (p.tile.kind && a.planes) {
+        if (!a.planes_ready &&
+            (e = lk_planes_launch(a.x, a.ldx, a.n_rows, a.K, type == LK_Q4_K, a.planes, st)) != hipSuccess)
+            return e;
+        if (a.ks == 0) a.ks = p.tile.ks;
+        if (a.ks > 1 && !a.part) return hipErrorInvalidValue;
+        e = lk_tile_launch(a, mode, p.tile, st);
+        if (deferred_ks) *deferred_ks = a.ks > 1 ? a.ks : 0;
+        if (e != hipSuccess || a.ks == 1 || deferred_ks) return e;
+        hipLaunchKernelGGL(lkg::gemm_reduce_kernel, dim3((a.N + 255) / 256, a.n_rows), dim3(256), 0, st, a, mode);
+        return hipGetLastError();
+    }
     // a wide, shallow matrix (the lm_head: one segment, no bias) without a K split: the kernel that
     // converts X once per block (bit-identical to gemm16_kernel)
     if (mode == LK_MV_STORE && a.nseg == 1 && !a.seg[0].bias && a.ks <= 1 && a.N >= LK_GEMM_WIDE_N &&
@@ -867,11 +913,9 @@ hipError_t lk_gemm_launch(LkGemmArgs a, int mode, hipStream_t st, uint32_t* defe
         if (type == LK_Q8_0) return one ? lkg::launch_wide_k<LK_Q8_0, 1>(a, st) : lkg::launch_wide_k<LK_Q8_0, 2>(a, st);
         return one ? lkg::launch_wide_k<LK_F16, 1>(a, st) : lkg::launch_wide_k<LK_F16, 2>(a, st);
     }
-    const LkGemmPlan p = lk_gemm_plan(type, a.N, a.K, a.n_rows, mode);
     if (a.ks == 0) a.ks = p.ks;
     if (a.ks > 1 && !a.part) return hipErrorInvalidValue;
     dim3 grid((a.N + 63) / 64, (a.n_rows + 16 * p.mb - 1) / (16 * p.mb), a.ks);
-    hipError_t e;
     switch (type) {
     case LK_Q8_0: e = lkg::launch_t<LK_Q8_0>(a, mode, p.mb, grid, st); break;
     case LK_F16: e = lkg::launch_t<LK_F16>(a, mode, p.mb, grid, st); break;

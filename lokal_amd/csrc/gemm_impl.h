@@ -102,5 +102,23 @@ __device__ __forceinline__ void dequant8(const Raw<WT>& R, int s, uint32_t kb, b
 
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
+// Epilogue of one output element: segment n (global index over segments).
+__device__ __forceinline__ void emit(const LkGemmArgs& a, int mode, uint32_t b, uint32_t n, float v, float u) {
+    if (mode == LK_MV_SWIGLU) {
+        a.seg[0].out[(size_t)b * a.ldy + n] = silu_mul(v, u);
+        return;
+    }
+    uint32_t si = 0, nb = 0;
+    while (si + 1 < a.nseg && n >= nb + a.seg[si].w.rows) {
+        nb += a.seg[si].w.rows;
+        si++;
+    }
+    const LkSeg& s = a.seg[si];
+    const uint32_t nl = n - nb;
+    if (s.bias) v += s.bias[nl];
+    float* o = s.out + (size_t)b * a.ldy + nl;
+    if (mode == LK_MV_ACC) *o += v;
+    else *o = v;
+}
 
 }  // namespace lkg

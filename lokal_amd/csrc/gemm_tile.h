@@ -1,0 +1,32 @@
+// gemm_tile.h -- the f16 planes of activation rows that gemm_tile.hip
+// multiplies: device code that writes them, and the buffer's layout.
+#pragma once
+#include "lkhip_common.h"
+
+// The power of two that brings a row's largest |x| (mx) into [2^14, 2^15)
+// (inv) and the one that undoes it (sc).  The exponent is kept where both
+// stay finite and normal; a row of zeros takes 2^15.
+__device__ __forceinline__ void lk_row_scale(float mx, float& inv, float& sc) {
+    int ex = 0;
+    (void)frexpf(mx, &ex);  // mx = f * 2^ex, f in [0.5, 1)
+    ex = mx == 0.f ? 0 : (ex < -100 ? -100 : (ex > 128 ? 128 : ex));
+    inv = ldexpf(1.0f, 15 - ex);
+    sc = ldexpf(1.0f, ex - 15);
+}
+
+// Stores 8 scaled values of row rr of row tile rt, columns 8g .. 8g+7, as f16
+// hi + lo where the MFMA operand lane that multiplies them reads them.
+__device__ __forceinline__ void lk_store_planes(void* xp, uint32_t rt, uint32_t rr, uint32_t nck, uint32_t g,
+                                                const float* v) {
+    typedef _Float16 lk_p8 __attribute__((ext_vector_type(8)));
+    lk_p8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        hi[e] = (_Float16)v[e];
+        lo[e] = (_Float16)(v[e] - (float)hi[e]);
+    }
+    const uint32_t p = g & 3, j = (p >> 1) | ((p & 1) << 1);  // columns 8p of the block sit in lanes j
+    lk_p8* o = (lk_p8*)xp + (((size_t)rt * nck * 4 + (g >> 2)) * 2) * 64 + j * 16 + rr;
+    o[0] = hi;
+    o[64] = lo;
+}

@@ -356,12 +356,53 @@ struct LkGemmArgs {
     uint32_t ldx, ldy;
     float* part;       // split-K partials [ks][n_rows][N or 2N]
     uint32_t ks;       // K splits (1: the epilogue runs in the GEMM kernel)
+    // gemm_tile.hip: workspace of lk_planes_bytes(n_rows, K) bytes for X as f16
+    // planes (null: the kernels that read X itself run), and whether it already
+    // holds them
+    void* planes;
+    uint32_t planes_ready;
+    const void* xp;    // set by lk_tile_launch
+    const float *xsc, *xsum;
 };
+// X as f16 planes: [row tile of 16][128-column chunk][32-column block][hi, lo][64 lanes][8 halves],
+// then each row's scale, then each row's scaled sums [row tile][block][16].
+struct LkPlanes {
+    void* xp;
+    float *xsc, *xsum;
+};
+inline size_t lk_planes_bytes(size_t n_rows, size_t K) {
+    const size_t rows = (n_rows + 15) / 16 * 16, kp = (K + 127) / 128 * 128;
+    return rows * kp * 4 + rows * 4 + rows * (kp / 32) * 4;
+}
+inline LkPlanes lk_planes_at(void* buf, size_t n_rows, size_t K) {
+    const size_t rows = (n_rows + 15) / 16 * 16, kp = (K + 127) / 128 * 128;
+    float* sc = (float*)((char*)buf + rows * kp * 4);
+    return LkPlanes{buf, sc, sc + rows};
+}
+// gemm_tile.hip's instances: output rows x activation rows of a block (SwiGLU: output rows of each of
+// gate and up), and its 64-column stages in LDS
+enum LkTileKind : uint32_t {
+    LK_TILE_NONE = 0,   // the tile kernel does not take the call
+    LK_TILE_SMALL = 1,  // 64 x 32, 4 stages
+    LK_TILE_MID = 2,    // 64 x 64, 2 stages (SwiGLU: as LK_TILE_LARGE)
+    LK_TILE_LARGE = 3,  // 128 x 64 (SwiGLU: 64 x 64), 2 stages
+    LK_TILE_SPLIT = 4   // 256 x 64 by 8 waves, 2 stages
+};
+struct LkTilePlan {
+    uint32_t kind;
+    uint32_t ks;
+};
+// X (rows ldx floats apart) into planes (lk_planes_bytes(n_rows, K)); sums: the Q4_K min term's row sums too
+hipError_t lk_planes_launch(const float* x, uint32_t ldx, uint32_t n_rows, uint32_t K, bool sums, void* planes,
+                            hipStream_t st);
+hipError_t lk_tile_launch(LkGemmArgs a, int mode, const LkTilePlan& p, hipStream_t st);
 // Plan: K splits for a launch and the partial floats it needs.
 struct LkGemmPlan {
     uint32_t ks;
     uint32_t mb;       // 16-row batch tiles per wave (1 or 2)
     size_t part_floats;
+    LkTilePlan tile;   // tile.kind != 0: gemm_tile.hip runs it, given a planes workspace
+    size_t plane_bytes;
 };
 LkGemmPlan lk_gemm_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_rows, int mode);
 // Checks the shape the GEMM assumes: N a multiple of 16 per segment, K of 32.

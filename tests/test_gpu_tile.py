@@ -1,0 +1,65 @@
+"""The many-row GEMM (gemm_tile.hip) through lkhip_matmul at the edges of its
+tiles and of the rule that picks them, against a float64 product of the
+oracle's dequantized weights.  Bound: every product of a 32-column block is
+exact, the block sums and the sums over blocks round in f32, so an output is
+off by at most (K / 32 + 40) * 2^-24 of the sum of |terms| (40: a block's own
+32 sums, the operand split's 2^-22, bias and scale)."""
+import numpy as np
+import pytest
+
+import oracle
+from lokal_amd import kernels as K
+from lokal_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # type, output rows, columns, activation rows
+    (synth.Q8_0, 6061, 64, 33),       # the fewest rows and columns; ragged outputs
+    (synth.Q8_0, 1553, 960, 131),     # an odd number of 64-column stages, ragged both ways
+    (synth.Q8_0, 200001, 32, 40),     # 32 columns: the general kernel (no whole stage)
+    (synth.Q8_0, 32741, 64, 65),      # 64 x 64 tiles
+    (synth.Q8_0, 131009, 64, 34),     # 128 x 64 tiles
+    (synth.Q8_0, 700, 4864, 300),     # K split over 8-wave blocks
+    (synth.F16, 3001, 608, 70),       # a half stage at the end
+    (synth.F16, 33000, 96, 67),
+    (synth.F16, 131072, 32, 33),
+    (synth.F16, 900, 1504, 250),
+    (synth.Q4_K, 4001, 256, 50),      # the smallest K
+    (synth.Q4_K, 32751, 256, 64),
+    (synth.Q4_K, 131007, 256, 33),
+    (synth.Q4_K, 1041, 2816, 257),    # an odd number of super-blocks, split
+]
+
+
+@pytest.mark.parametrize("t,rows,cols,n", CASES)
+def test_matmul_tiles_match_float64(t, rows, cols, n):
+    data = synth.gen_weight(t, 11, f"w{rows}x{cols}", rows, cols).data
+    ref = oracle.dequant_row(t, data, rows * cols).reshape(rows, cols).astype(np.float64)
+    rng = np.random.default_rng(rows + cols + n)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[1] = 0.0                  # a row of zeros
+    x[2] *= np.float32(1e-30)   # rows far from 1, and one of mixed magnitudes
+    x[3] *= np.float32(1e30)
+    x[4, ::3] *= np.float32(1e-9)
+    x[5] = 0.0                  # one-hot: the weight column, bit for bit
+    x[5, cols - 1] = 1.0
+    bias = rng.standard_normal(rows).astype(np.float32)
+    ldx, ldy = cols + 4, rows + 3
+    xp = np.full((n, ldx), 7.0, np.float32)
+    xp[:, :cols] = x
+    w = K.Weight(t, rows, cols, data)
+    xd, bd = K.DeviceArray.from_numpy(xp), K.DeviceArray.from_numpy(bias)
+    y = K.DeviceArray((n, ldy))
+    y.upload(np.full((n, ldy), 3.0, np.float32))
+    K.matmul(w, xd, n, y, ldx=ldx, ldy=ldy)
+    got = y.numpy()
+    assert np.all(got[:, rows:] == 3.0)
+    assert np.array_equal(got[5, :rows], ref[:, cols - 1].astype(np.float32))
+    want = x.astype(np.float64) @ ref.T
+    scale = np.abs(x).astype(np.float64) @ np.abs(ref).T
+    bar = (cols / 32 + 40) * 2.0 ** -24
+    assert np.max(np.abs(got[:, :rows] - want) / (scale + 1e-300)) < bar
+    # accumulate, and a bias
+    K.matmul(w, xd, n, y, bias=bd, accumulate=True, ldx=ldx, ldy=ldy)
+    twice = y.numpy()[:, :rows]
+    assert np.max(np.abs(twice - (2 * want + bias)) / (2 * scale + np.abs(bias) + 1e-300)) < bar
