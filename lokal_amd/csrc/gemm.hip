@@ -818,7 +818,7 @@ static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_ro
     LkTilePlan p{};
     const bool sw = mode == LK_MV_SWIGLU;
     if (n_rows < LK_TILE_MIN_ROWS || (uint64_t)N * (sw ? 2 : 1) * n_rows < LK_TILE_MIN_SUMS) return p;
-    if (!lkg::gemm16_on(type) || (type == LK_Q8_0 && K % 64)) return p;  // whole 64-column stages of block scales
+    if (!lkg::gemm16_on(type == LK_Q8_SM ? (uint32_t)LK_Q8_0 : type) || ((type == LK_Q8_0 || type == LK_Q8_SM) && K % 64)) return p;  // whole 64-column stages of block scales
     // 32-bit offsets inside a block's rows and the planes
     if (lk_planes_bytes(n_rows, K) >> 32 || (uint64_t)K * 64 >> 31) return p;
     const uint32_t nck = (K + lkg::KC - 1) / lkg::KC;
@@ -837,7 +837,7 @@ static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_ro
         if (p.kind == LK_TILE_SMALL) ks = 192 / blocks(64, 32);
     } else if (blocks(128, 64) >= 1024) {
         p.kind = LK_TILE_LARGE;
-    } else if (blocks(64, 64) >= 512) {
+    } else if (blocks(64, 64) >= (K <= 1024 ? 512 : 320)) {
         p.kind = LK_TILE_MID;
     } else if (K <= 1024) {
         p.kind = LK_TILE_SMALL;
@@ -893,7 +893,7 @@ hipError_t lk_gemm_launch(LkGemmArgs a, int mode, hipStream_t st, uint32_t* defe
     hipError_t e;
     if (p.tile.kind && a.planes) {
         if (!a.planes_ready &&
-            (e = lk_planes_launch(a.x, a.ldx, a.n_rows, a.K, type == LK_Q4_K, a.planes, st)) != hipSuccess)
+            (e = lk_planes_launch(a.x, a.ldx, a.n_rows, a.K, lk_planes_sums(type), a.planes, st)) != hipSuccess)
             return e;
         if (a.ks == 0) a.ks = p.tile.ks;
         if (a.ks > 1 && !a.part) return hipErrorInvalidValue;

@@ -58,11 +58,11 @@ __device__ __forceinline__ h8 bytes_h8(uint32_t w0, uint32_t w1, float off) {
 
 template <int WT>
 __device__ __forceinline__ uint32_t row_bytes(uint32_t K) {
-    return WT == LK_Q8_0 ? K : WT == LK_F16 ? 2 * K : K / 2;
+    return WT == LK_Q8_0 || WT == LK_Q8_SM ? K : WT == LK_F16 ? 2 * K : K / 2;
 }
 template <int WT>
 __device__ __forceinline__ uint32_t aux_bytes(uint32_t K) {
-    return WT == LK_Q8_0 ? K / 16 : WT == LK_F16 ? 0 : K / 16;
+    return WT == LK_Q8_SM ? K / 2 : WT == LK_F16 ? 0 : K / 16;
 }
 
 // 16 (4) bytes per lane from global memory straight to LDS: lane l's to dst + 16 l (4 l)
@@ -82,12 +82,13 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
     constexpr int NO = SW ? NT / 2 : NT;  // output tiles of a wave
     // LDS of one 64-column stage: X planes [row tile][block of 2][plane][lane] for the
     // block, then each wave's own weights in operand order, block scales or
-    // super-block heads, and (Q4_K) the rows' sums; a ring of RING stages
-    constexpr int WP = WT == LK_Q8_0 ? NT : WT == LK_F16 ? 2 * NT : (NT + 1) / 2;  // weight loads of a wave per stage
-    constexpr int AUX = WT == LK_Q8_0 ? 16 : WT == LK_Q4_K ? 64 + 16 : 0;    // u4 per wave
+    // super-block heads, and (types with mins) the rows' sums; a ring of RING stages
+    constexpr bool SM = WT == LK_Q8_SM, MIN = WT == LK_Q4_K || SM;
+    constexpr int WP = WT == LK_Q8_0 || SM ? NT : WT == LK_F16 ? 2 * NT : (NT + 1) / 2;  // weight loads of a wave per stage
+    constexpr int AUX = WT == LK_Q8_0 ? 16 : MIN ? 64 + 16 : 0;              // u4 per wave
     constexpr int XU = MT * 256, WU = NW * WP * 64, SU = XU + WU + NW * AUX, XI = MT * 4 / NW;
-    constexpr int OPS = XI + WP + (WT == LK_Q8_0 ? 1 : WT == LK_Q4_K ? 2 : 0);  // loads of a wave per stage
-    static_assert(16 * NT <= 64 && XI >= 1, "one lane per weight row; an X load per wave");
+    constexpr int OPS = XI + WP + (WT == LK_Q8_0 ? 1 : MIN ? 2 : 0);  // loads of a wave per stage
+    static_assert(16 * NT <= 64 && XI >= 1 && (!SM || NT <= 2), "one lane per weight row; an X load per wave");
     static_assert((RING & (RING - 1)) == 0 && (RING - 2) * OPS <= 63, "slots by mask; vmcnt holds 6 bits");
     __shared__ __align__(16) u4 ring[RING][SU];
     const int lane = threadIdx.x & 63;
@@ -129,14 +130,18 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
             if (t % 2 == 0 || lane >= 32) wq[t / 2] = v;
             ow[t] = 0;
         } else {
-            ow[t] = lr * row_bytes<WT>(K) + (WT == LK_Q8_0 ? 16 * j : 32 * (j & 1) + 16 * (j >> 1));
+            ow[t] = lr * row_bytes<WT>(K) + (WT == LK_F16 ? 32 * (j & 1) + 16 * (j >> 1) : 16 * j);
         }
         if constexpr (AUX != 0) {
             const uint8_t* v = sg->w.aux + (size_t)l0 * aux_bytes<WT>(K) + lr * aux_bytes<WT>(K);
-            if (t == 0 || j % NT == (uint32_t)t) wa = v;
+            if constexpr (SM) {  // 32 bytes (4 groups) of a row per stage: 16 per lane, lanes 32.. the second tile
+                if (t == 0 || lane >= 32) wa = v + 16 * (j & 1);
+            } else {
+                if (t == 0 || j % NT == (uint32_t)t) wa = v;
+            }
         }
     }
-    // row tile of the wave's i-th X load, and (Q4_K) this lane's source of the rows' sums: row tile wave % MT
+    // row tile of the wave's i-th X load, and (types with mins) the source of the rows' sums: row tile wave % MT
     const uint8_t* xb[XI];
 #pragma unroll
     for (int i = 0; i < XI; i++) {
@@ -144,9 +149,9 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
         xb[i] = (const uint8_t*)a.xp + ((size_t)rt * nck * 8 + q % 4) * 1024;
     }
     const float* xq = nullptr;
-    if constexpr (WT == LK_Q4_K) {
+    if constexpr (MIN) {
         const uint32_t rt = rt0 + wave % MT < RT ? rt0 + wave % MT : RT - 1;
-        xq = a.xsum + (size_t)rt * nck * 64;
+        xq = a.xsum + (size_t)rt * nck * 128 + lane;
     }
     const uint32_t l16 = lane * 16;
     // all loads of stage s (of this block's range) into its ring slot
@@ -164,15 +169,20 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
                     const uint32_t k = g * 64 + 32 * b;  // past K: column 0, multiplied by zero planes
                     dma16(wd[t] + (size_t)2 * (k < K ? k : 0) + ow[t], ws + (2 * t + b) * 64);
                 }
-        } else if constexpr (WT == LK_Q8_0) {
+        } else if constexpr (WT == LK_Q8_0 || SM) {
 #pragma unroll
             for (int t = 0; t < NT; t++) dma16(wd[t] + (size_t)g * 64 + ow[t], ws + t * 64);
-            dma4(wa + g * 4, as);
+            if constexpr (SM) {
+                dma16(wa + g * 32, as);
+                dma4(xq + (size_t)g * 64, as + 64);
+            } else {
+                dma4(wa + g * 4, as);
+            }
         } else {
 #pragma unroll
             for (int t = 0; t < WP; t++) dma16((const uint8_t*)wq[t] + g * 32, ws + t * 64);
             dma16(wa + (g >> 2) * 16, as);
-            dma4(xq + (size_t)g * 32 + (lane & 31), as + 64);
+            dma4(xq + (size_t)g * 64, as + 64);
         }
     };
 
@@ -181,7 +191,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
     for (int t = 0; t < NT; t++)
 #pragma unroll
         for (int m = 0; m < MT; m++) y[t][m] = f4{0.f, 0.f, 0.f, 0.f};
-    float mn[NT], xs[WT == LK_Q4_K ? MT : 1];  // Q4_K: -m1 and the sums of sub-block j of the chunk
+    // -m and the rows' sums: Q4_K of sub-block j of the chunk, Q8_SM of 16-column group j of the stage
+    float mn[NT], xs[MIN ? MT : 1];
 #pragma unroll
     for (uint32_t s = 0; s < RING - 1; s++)
         if (s < S) stage_load(s, ring[s]);
@@ -197,7 +208,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
         const u4* const slot = ring[RING == 2 ? h : s % RING];
         const u4* const ws = slot + XU + wave * WP * 64;
         const u4* const as = slot + XU + WU + wave * AUX;
-        float d[NT][2];
+        float d[NT][SM ? 4 : 2];  // scale of each 32-column block (Q8_SM: of each 16 columns)
         u4 q[NT][WT == LK_F16 ? 2 : 1];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -205,6 +216,14 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
                 q[t][0] = ws[t * 64 + lane];
                 const uint32_t v = ((const uint32_t*)as)[t * 16 + c16];
                 d[t][0] = lk_h2f((uint16_t)(v & 0xFFFF)), d[t][1] = lk_h2f((uint16_t)(v >> 16));
+                swap_blocks(q[t][0]);
+            } else if constexpr (SM) {
+                q[t][0] = ws[t * 64 + lane];
+                const u4 g0 = as[t * 32 + c16], g1 = as[t * 32 + 16 + c16];  // (s, m) of groups 0, 1 and 2, 3
+                d[t][0] = __uint_as_float(g0[0]), d[t][1] = __uint_as_float(g0[2]);
+                d[t][2] = __uint_as_float(g1[0]), d[t][3] = __uint_as_float(g1[2]);
+                const uint32_t me = j < 2 ? ((j & 1) ? g0[3] : g0[1]) : ((j & 1) ? g1[3] : g1[1]);
+                mn[t] = -__uint_as_float(me);
                 swap_blocks(q[t][0]);
             } else if constexpr (WT == LK_F16) {
                 q[t][0] = ws[2 * t * 64 + lane];
@@ -223,12 +242,16 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
                 mn[t] = h == 0 || j >= 2 ? mv : mn[t];  // stage h holds sub-blocks 2h, 2h + 1
             }
         }
-        if constexpr (WT == LK_Q4_K) {
+        if constexpr (MIN) {
 #pragma unroll
             for (int m = 0; m < MT; m++) {
-                const float* sm = (const float*)(slot + XU + WU + (m % 4) * AUX + 64);
-                const float v = sm[(j & 1) * 16 + c16];
-                xs[m] = h == 0 || j >= 2 ? v : xs[m];
+                const float* sm = (const float*)(slot + XU + WU + m * AUX + 64);  // sums of 16 columns: [group][row]
+                if constexpr (SM) {
+                    xs[m] = sm[j * 16 + c16];
+                } else {
+                    const float v = sm[(j & 1) * 32 + c16] + sm[(j & 1) * 32 + 16 + c16];
+                    xs[m] = h == 0 || j >= 2 ? v : xs[m];
+                }
             }
         }
         // both blocks' X operands are read before the first product, so LDS
@@ -246,12 +269,43 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
             h8 w[NT];
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                if constexpr (WT == LK_Q8_0)
+                if constexpr (WT == LK_Q8_0 || SM)
                     w[t] = bytes_h8(q[t][0][2 * b] ^ 0x80808080u, q[t][0][2 * b + 1] ^ 0x80808080u, 1152.0f);
                 else if constexpr (WT == LK_F16)
                     w[t] = __builtin_bit_cast(h8, q[t][b]);
                 else
                     w[t] = bytes_h8((q[t][0][0] >> (4 * b)) & 0x0F0F0F0Fu, (q[t][0][1] >> (4 * b)) & 0x0F0F0F0Fu, 1024.0f);
+            }
+            if constexpr (SM) {
+                // a 32-column block holds two groups with scales of their own: lanes j = 0, 2 the
+                // first, 1, 3 the second, the other's weights zero
+                const uint32_t keep0 = (j & 1) ? 0u : ~0u;
+#pragma unroll
+                for (int gq = 0; gq < 2; gq++) {
+                    h8 wg[NT];
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        u4 v = __builtin_bit_cast(u4, w[t]);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[e] &= gq ? ~keep0 : keep0;
+                        wg[t] = __builtin_bit_cast(h8, v);
+                    }
+                    f4 D[MT][NT];
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+#pragma unroll
+                        for (int p = 0; p < 2; p++)
+#pragma unroll
+                            for (int t = 0; t < NT; t++)
+                                D[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][m][p], wg[t], p ? D[m][t] : f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+#pragma unroll
+                        for (int t = 0; t < NT; t++)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) y[t][m][i] = fmaf(d[t][2 * b + gq], D[m][t][i], y[t][m][i]);
+                }
+                continue;
             }
             f4 D[MT][NT];
 #pragma unroll
@@ -281,8 +335,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
         for (int t = 0; t < NT; t++)
 #pragma unroll
             for (int m = 0; m < MT; m++) asm volatile("" : "+v"(y[t][m]));
-        if constexpr (WT == LK_Q4_K && h == 1) {
-            // minus m1 * sum(x) per sub-block: the chunk's four are one f32 MFMA
+        if constexpr (SM || (WT == LK_Q4_K && h == 1)) {
+            // minus m * sum(x) per sub-block or group: four of them are one f32 MFMA
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
@@ -360,8 +414,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
 // Four activation rows per block, WPR waves each (rows past the last, up to a
 // whole 16-row tile, are zero): the row's power-of-two scale, its f16 planes
 // in MFMA order [row tile][chunk][block][plane][lane], the scale that undoes
-// it, and with `xsum` the row's scaled sum over every 32-column block (the Q4_K
-// min term).  A lane holds its G groups of 8 columns from the load to the
+// it, and with `xsum` the row's scaled sum over every 16 columns (the Q4_K and Q8_SM
+// min terms).  A lane holds its G groups of 8 columns from the load to the
 // store (G = 0: a row too wide for that is read twice).  The four rows' 16-byte
 // pieces of a 64-byte line leave one CU together; one row per block
 // wrote each line from four XCDs.  512 rows of 4864: 11.0 -> 7.6 us.
@@ -419,8 +473,7 @@ __global__ __launch_bounds__(256 * WPR) void x_planes_kernel(const float* __rest
         if (xsum) {
             float s = ((o[0] + o[1]) + (o[2] + o[3])) + ((o[4] + o[5]) + (o[6] + o[7]));
             s += __shfl_xor(s, 1, 64);
-            s += __shfl_xor(s, 2, 64);
-            if (g % 4 == 0 && g < nck * 16) xsum[((size_t)rt * nck * 4 + g / 4) * 16 + rr] = s;
+            if (g % 2 == 0 && g < nck * 16) xsum[((size_t)rt * nck * 8 + g / 2) * 16 + rr] = s;
         }
     };
     if constexpr (G != 0) {
@@ -446,7 +499,7 @@ static hipError_t launch(const LkGemmArgs& a, int mode, hipStream_t st) {
 template <int WT>
 static hipError_t launch_t(const LkGemmArgs& a, int mode, uint32_t kind, hipStream_t st) {
     if (mode == LK_MV_SWIGLU) {
-        if (kind == LK_TILE_SMALL) return launch<WT, 4, 2, 2, true, WT == LK_F16 ? 2 : 4>(a, mode, st);
+        if (kind == LK_TILE_SMALL) return launch<WT, 4, 2, 2, true, WT == LK_F16 || WT == LK_Q8_SM ? 2 : 4>(a, mode, st);
         return launch<WT, 4, 2, 4, true, 2>(a, mode, st);
     }
     switch (kind) {
@@ -488,6 +541,7 @@ hipError_t lk_tile_launch(LkGemmArgs a, int mode, const LkTilePlan& p, hipStream
     case LK_Q8_0: return lkt::launch_t<LK_Q8_0>(a, mode, p.kind, st);
     case LK_F16: return lkt::launch_t<LK_F16>(a, mode, p.kind, st);
     case LK_Q4_K: return lkt::launch_t<LK_Q4_K>(a, mode, p.kind, st);
+    case LK_Q8_SM: return lkt::launch_t<LK_Q8_SM>(a, mode, p.kind, st);
     default: return hipErrorInvalidValue;
     }
 }

@@ -365,14 +365,16 @@ struct LkGemmArgs {
     const float *xsc, *xsum;
 };
 // X as f16 planes: [row tile of 16][128-column chunk][32-column block][hi, lo][64 lanes][8 halves],
-// then each row's scale, then each row's scaled sums [row tile][block][16].
+// then each row's scale, then each row's scaled sums over 16 columns [row tile][16 columns][16 rows].
 struct LkPlanes {
     void* xp;
     float *xsc, *xsum;
 };
+// whether a weight type's product reads the sums
+inline bool lk_planes_sums(uint32_t type) { return type == LK_Q4_K || type == LK_Q8_SM; }
 inline size_t lk_planes_bytes(size_t n_rows, size_t K) {
     const size_t rows = (n_rows + 15) / 16 * 16, kp = (K + 127) / 128 * 128;
-    return rows * kp * 4 + rows * 4 + rows * (kp / 32) * 4;
+    return rows * kp * 4 + rows * 4 + rows * (kp / 16) * 4;
 }
 inline LkPlanes lk_planes_at(void* buf, size_t n_rows, size_t K) {
     const size_t rows = (n_rows + 15) / 16 * 16, kp = (K + 127) / 128 * 128;
@@ -392,7 +394,7 @@ struct LkTilePlan {
     uint32_t kind;
     uint32_t ks;
 };
-// X (rows ldx floats apart) into planes (lk_planes_bytes(n_rows, K)); sums: the Q4_K min term's row sums too
+// X (rows ldx floats apart) into planes (lk_planes_bytes(n_rows, K)); sums: the row sums of Q4_K's and Q8_SM's min terms too
 hipError_t lk_planes_launch(const float* x, uint32_t ldx, uint32_t n_rows, uint32_t K, bool sums, void* planes,
                             hipStream_t st);
 hipError_t lk_tile_launch(LkGemmArgs a, int mode, const LkTilePlan& p, hipStream_t st);

@@ -28,6 +28,11 @@ CASES = [  # type, output rows, columns, activation rows
     (synth.Q4_K, 32751, 256, 64),
     (synth.Q4_K, 131007, 256, 33),
     (synth.Q4_K, 1041, 2816, 257),    # an odd number of super-blocks, split
+    (synth.Q6_K, 6061, 256, 33),      # 16-column groups of scales (and, Q5_K, mins)
+    (synth.Q6_K, 1553, 768, 131),
+    (synth.Q6_K, 131007, 256, 33),
+    (synth.Q5_K, 32751, 256, 64),
+    (synth.Q5_K, 1041, 2816, 257),
 ]
 
 
