@@ -825,23 +825,32 @@ static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_ro
     auto blocks = [&](uint32_t bn, uint32_t bm) { return ((N + bn - 1) / bn) * ((n_rows + bm - 1) / bm); };
     // The largest tile that leaves every CU several waves: a lone wave per SIMD
     // issues a vector instruction every 7 cycles, three or four together one
-    // every 3.5-4, and a stage is bound by that.  Few tiles: the small one, K
-    // split over the grid when even that leaves CUs without a block; a deep K
-    // amortises 8-wave blocks that share X, with K split over 256 of them.
-    // Q8_0 4864 x 896, 512 rows, by kind (kernel us): small 22.9, mid 19.1, large
-    // 21.3, split (8) 31.8; 896 x 896: 9.2 / 11.5 / 14.5 / 9.7; 896 x 4864:
-    // 32.1 / 47.4 / 60.1 / 20.0; 151936 x 896, 64 rows: 72 / 55 / 47 / 110.
+    // every 3.5-4, and a stage is bound by that.  Few tiles: small ones whose
+    // K is split between two groups of waves (small) or four (deep, as long as its
+    // 16-wave blocks all run at once), and K split over the grid too when CUs
+    // are left without a block; a deep K amortises 8-wave blocks that share X,
+    // with K split over 256 of them.  F16 has no block scales to apply and does
+    // best with one group and four stages in flight, also at a deep K; Q8_SM does
+    // twice the products per weight, so more of its waves beat larger tiles.
+    // Kernel us (with the reduction of a split), small / deep / mid / split:
+    //   Q8_0 896 x 896, 512 rows: 9.1 / 8.2 / 11.5 / 13.7; 1152 x 896: 10.3 / 14.4 / 11.6;
+    //   4864 x 896: 22.9 / - / 19.1 / 31.8 (large 21.3); 896 x 4864: 32 / 27.9 / 47 / 25.4;
+    //   Q4_K 2048 x 2048, 256 rows: 19 / 16.2 / - / 18.8; 2560 x 2048: 22.4 / 28.5 / - / 21;
+    //   Q8_SM 2048 x 2048, 256 rows: 19.2 / 17.7 / 28.8 / 21.5; 5632 x 2048: 39.1 / - / 43.7;
+    //   F16 576 x 576, 512 rows: 6.5 / 7.2 / 9.4; 576 x 1536: 11.4 / 13.4 / 18.6 / 16.4;
+    //   Q8_0 151936 x 896, 64 rows: 72 / - / 55 / 110 (large 47).
+    const uint32_t small = blocks(64, 32);
     uint32_t ks = 1;
     if (sw) {
         p.kind = blocks(64, 64) >= 256 ? LK_TILE_LARGE : LK_TILE_SMALL;
-        if (p.kind == LK_TILE_SMALL) ks = 192 / blocks(64, 32);
+        if (p.kind == LK_TILE_SMALL) ks = 192 / small;
     } else if (blocks(128, 64) >= 1024) {
         p.kind = LK_TILE_LARGE;
     } else if (blocks(64, 64) >= (K <= 1024 ? 512 : 320)) {
-        p.kind = LK_TILE_MID;
-    } else if (K <= 1024) {
-        p.kind = LK_TILE_SMALL;
-        ks = 192 / blocks(64, 32);
+        p.kind = type == LK_Q8_SM ? LK_TILE_SMALL : LK_TILE_MID;
+    } else if (K <= 1024 || (K <= 2048 && (type == LK_F16 ? small >= 128 : small >= 192 && small <= 256))) {
+        p.kind = small > 256 || type == LK_F16 ? LK_TILE_SMALL : LK_TILE_DEEP;
+        ks = 192 / small;
     } else {
         p.kind = LK_TILE_SPLIT;
         ks = (256 + blocks(256, 64) - 1) / blocks(256, 64);

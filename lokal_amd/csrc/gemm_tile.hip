@@ -13,7 +13,9 @@
 // us = 94 TFLOP/s; here 20.5 us + 4.9 for the planes = 175 TFLOP/s).
 //
 // gemm_tile_kernel: a block of NW waves takes 16 NT NW weight rows x 16 MT
-// activation rows over a range of K, 64 columns (a stage) at a time.  Every
+// activation rows over a range of K, 64 columns (a stage) at a time; KG such
+// groups of waves share a block's tile, each with every KG-th pair of stages, and
+// add up through LDS (four groups, 896 x 896 Q8_0, 512 rows: 9.3 -> 8.2 us).  Every
 // load goes straight to LDS (global_load_lds, no registers, RING stages deep):
 // the X planes shared by the block, and each wave's own weight rows and scales
 // in the order it reads them back.  X is the MFMA's A operand and W its B, so a
@@ -75,10 +77,10 @@ __device__ __forceinline__ void dma4(const void* src, void* dst) {
     __builtin_amdgcn_global_load_lds((gptr)src, (lptr)dst, 4, 0, 0);
 }
 
-template <int WT, int NW, int NT, int MT, bool SW, uint32_t RING>
+template <int WT, int NW, int NT, int MT, bool SW, uint32_t RING, int KG>
 // two blocks' waves per SIMD: 256 registers, which also keeps the products out of the accumulation
 // registers (moving them back cost 64 instructions a stage)
-__global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs a, int mode) {
+__global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemmArgs a, int mode) {
     constexpr int NO = SW ? NT / 2 : NT;  // output tiles of a wave
     // LDS of one 64-column stage: X planes [row tile][block of 2][plane][lane] for the
     // block, then each wave's own weights in operand order, block scales or
@@ -90,15 +92,26 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
     constexpr int OPS = XI + WP + (WT == LK_Q8_0 ? 1 : MIN ? 2 : 0);  // loads of a wave per stage
     static_assert(16 * NT <= 64 && XI >= 1 && (!SM || NT <= 2), "one lane per weight row; an X load per wave");
     static_assert((RING & (RING - 1)) == 0 && (RING - 2) * OPS <= 63, "slots by mask; vmcnt holds 6 bits");
-    __shared__ __align__(16) u4 ring[RING][SU];
+    __shared__ __align__(16) u4 rings[KG][RING][SU];
     const int lane = threadIdx.x & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // KG groups of NW waves take the block's chunks in turn, each with a ring of its own
+    const uint32_t kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / NW;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % NW;
+    u4(*const ring)[SU] = rings[kg];
     const uint32_t j = (uint32_t)lane >> 4, c16 = (uint32_t)lane & 15;
     const uint32_t K = a.K, nck = (K + 127) / 128, nst = (K + 63) / 64;
     const uint32_t per = (nck + a.ks - 1) / a.ks;
     const uint32_t s_begin = 2 * blockIdx.z * per;
     const uint32_t s_end = s_begin + 2 * per < nst ? s_begin + 2 * per : nst;
-    const uint32_t S = s_begin < s_end ? s_end - s_begin : 0;
+    const uint32_t ST = s_begin < s_end ? s_end - s_begin : 0;  // the block's stages
+    // the group's i-th pair of stages is the block's pair kg + i KG
+    auto stage_of = [&](uint32_t s) { return KG == 1 ? s : (s >> 1) * (2 * KG) + 2 * kg + (s & 1); };
+    uint32_t S = ST;
+    if constexpr (KG > 1) {
+        const uint32_t pairs = ST / 2, left = ST % 2;  // an odd last stage goes to the group next in turn
+        S = pairs / KG * 2 + (pairs % KG > kg ? 2 : 0) + (left && pairs % KG == kg ? 1 : 0);
+    }
+    const uint32_t SI = KG == 1 ? S : (ST + 2 * KG - 1) / (2 * KG) * 2;  // iterations of every group (barriers)
     const uint32_t RT = (a.n_rows + 15) / 16, rt0 = blockIdx.y * MT;
 
     // The wave's tiles: a uniform base (the tile's first row) and this lane's
@@ -156,7 +169,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
     const uint32_t l16 = lane * 16;
     // all loads of stage s (of this block's range) into its ring slot
     auto stage_load = [&](uint32_t s, u4* slot) {
-        const uint32_t g = s_begin + s;  // 64-column group
+        const uint32_t g = s_begin + stage_of(s);  // 64-column group
 #pragma unroll
         for (int i = 0; i < XI; i++) dma16(xb[i] + (size_t)g * 4096 + l16, slot + (wave * XI + i) * 64);
         u4* const ws = slot + XU + wave * WP * 64;
@@ -205,6 +218,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
         if (RING > 2 && s + RING - 2 < S) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RING - 2) * OPS) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (s + RING - 1 < S) stage_load(s + RING - 1, ring[RING == 2 ? h ^ 1 : (s + RING - 1) % RING]);
+        if (KG > 1 && s >= S) return;  // the barrier only
         const u4* const slot = ring[RING == 2 ? h : s % RING];
         const u4* const ws = slot + XU + wave * WP * 64;
         const u4* const as = slot + XU + WU + wave * AUX;
@@ -236,7 +250,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
                 const u4 hd = as[t * 16 + c16];
                 const float ds = lk_h2f((uint16_t)(hd[0] & 0xFFFF)), dm = lk_h2f((uint16_t)(hd[0] >> 16));
                 uint32_t sc0, sc1, m0, m1;
-                lk::scale_min_k4_pair((s_begin + s) & 3, hd[1], hd[2], hd[3], sc0, m0, sc1, m1);
+                lk::scale_min_k4_pair((s_begin + stage_of(s)) & 3, hd[1], hd[2], hd[3], sc0, m0, sc1, m1);
                 d[t][0] = __fmul_rn(ds, (float)sc0), d[t][1] = __fmul_rn(ds, (float)sc1);
                 const float mv = -__fmul_rn(dm, (float)((j & 1) ? m1 : m0));
                 mn[t] = h == 0 || j >= 2 ? mv : mn[t];  // stage h holds sub-blocks 2h, 2h + 1
@@ -345,9 +359,28 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tile_kernel(const LkGemmArgs 
         }
     };
 #pragma unroll 1
-    for (uint32_t s = 0; s < S; s += 2) {
+    for (uint32_t s = 0; s < SI; s += 2) {
         stage(s, std::integral_constant<uint32_t, 0>{});
-        if (s + 1 < S) stage(s + 1, std::integral_constant<uint32_t, 1>{});
+        if (KG > 1 || s + 1 < S) stage(s + 1, std::integral_constant<uint32_t, 1>{});
+    }
+    if constexpr (KG > 1) {
+        // the groups' sums, through LDS, into group 0's in turn
+        f4* const acc = (f4*)&rings[0][0][0];
+        static_assert(sizeof(rings) >= (size_t)(KG - 1) * NW * NT * MT * 64 * 16, "the sums fit the rings");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (kg)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) acc[((((kg - 1) * NW + wave) * NT + t) * MT + m) * 64 + lane] = y[t][m];
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (kg) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; g++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) y[t][m] += acc[(((g * NW + wave) * NT + t) * MT + m) * 64 + lane];
     }
 
     // lane: rows 4j + i of each row tile, output on[t] + c16.  A K split leaves
@@ -487,26 +520,32 @@ __global__ __launch_bounds__(256 * WPR) void x_planes_kernel(const float* __rest
     }
 }
 
-template <int WT, int NW, int NT, int MT, bool SW, uint32_t RING>
+template <int WT, int NW, int NT, int MT, bool SW, uint32_t RING, int KG = 1>
 static hipError_t launch(const LkGemmArgs& a, int mode, hipStream_t st) {
     constexpr uint32_t BN = 16 * NW * (SW ? NT / 2 : NT);
     const dim3 grid((a.N + BN - 1) / BN, (a.n_rows + 16 * MT - 1) / (16 * MT), a.ks);
-    hipLaunchKernelGGL((gemm_tile_kernel<WT, NW, NT, MT, SW, RING>), grid, dim3(64 * NW), 0, st, a, mode);
+    hipLaunchKernelGGL((gemm_tile_kernel<WT, NW, NT, MT, SW, RING, KG>), grid, dim3(64 * NW * KG), 0, st, a, mode);
     return hipGetLastError();
 }
 
 // The instances tile_plan chooses from, by its names for them.
 template <int WT>
 static hipError_t launch_t(const LkGemmArgs& a, int mode, uint32_t kind, hipStream_t st) {
+    constexpr bool ONE = WT == LK_F16;  // no wave groups
     if (mode == LK_MV_SWIGLU) {
-        if (kind == LK_TILE_SMALL) return launch<WT, 4, 2, 2, true, WT == LK_F16 || WT == LK_Q8_SM ? 2 : 4>(a, mode, st);
+        if (kind == LK_TILE_SMALL) return launch<WT, 4, 2, 2, true, 2, ONE ? 1 : 2>(a, mode, st);
         return launch<WT, 4, 2, 4, true, 2>(a, mode, st);
     }
     switch (kind) {
-    case LK_TILE_SMALL: return launch<WT, 4, 1, 2, false, 4>(a, mode, st);
-    case LK_TILE_MID: return launch<WT, 4, 1, 4, false, 2>(a, mode, st);
+    case LK_TILE_SMALL: return launch<WT, 4, 1, 2, false, ONE ? 4 : 2, ONE ? 1 : 2>(a, mode, st);
+    case LK_TILE_MID:
+        if constexpr (WT != LK_Q8_SM) return launch<WT, 4, 1, 4, false, 2>(a, mode, st);
+        return hipErrorInvalidValue;
     case LK_TILE_LARGE: return launch<WT, 4, 2, 4, false, 2>(a, mode, st);
     case LK_TILE_SPLIT: return launch<WT, 8, 2, 4, false, 2>(a, mode, st);
+    case LK_TILE_DEEP:
+        if constexpr (!ONE) return launch<WT, 4, 1, 2, false, 2, 4>(a, mode, st);
+        return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
 }

@@ -385,10 +385,11 @@ inline LkPlanes lk_planes_at(void* buf, size_t n_rows, size_t K) {
 // gate and up), and its 64-column stages in LDS
 enum LkTileKind : uint32_t {
     LK_TILE_NONE = 0,   // the tile kernel does not take the call
-    LK_TILE_SMALL = 1,  // 64 x 32, 4 stages
-    LK_TILE_MID = 2,    // 64 x 64, 2 stages (SwiGLU: as LK_TILE_LARGE)
+    LK_TILE_SMALL = 1,  // 64 x 32, two wave groups of 2 stages (F16: one of 4)
+    LK_TILE_MID = 2,    // 64 x 64, 2 stages (SwiGLU: as LK_TILE_LARGE; not Q8_SM)
     LK_TILE_LARGE = 3,  // 128 x 64 (SwiGLU: 64 x 64), 2 stages
-    LK_TILE_SPLIT = 4   // 256 x 64 by 8 waves, 2 stages
+    LK_TILE_SPLIT = 4,  // 256 x 64 by 8 waves, 2 stages
+    LK_TILE_DEEP = 5    // 64 x 32, four wave groups of 2 stages (not SwiGLU, not F16)
 };
 struct LkTilePlan {
     uint32_t kind;

@@ -33,6 +33,11 @@ CASES = [  # type, output rows, columns, activation rows
     (synth.Q6_K, 131007, 256, 33),
     (synth.Q5_K, 32751, 256, 64),
     (synth.Q5_K, 1041, 2816, 257),
+    (synth.Q8_0, 4101, 832, 131),     # two wave groups, 13 stages between them
+    (synth.Q6_K, 4101, 256, 131),
+    (synth.Q8_0, 905, 192, 250),      # four wave groups for three stages
+    (synth.Q4_K, 1041, 1792, 380),    # four wave groups, a deep K
+    (synth.F16, 1041, 1504, 380),     # one group, a deep K
 ]
 
 
