@@ -278,6 +278,7 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
 #pragma unroll
                 for (int p = 0; p < 2; p++)
                     xf[b][m][p] = __builtin_bit_cast(h8, slot[(m * 4 + b * 2 + p) * 64 + lane]);
+        f4 D[MT][NT];
 #pragma unroll
         for (int b = 0; b < 2; b++) {
             h8 w[NT];
@@ -304,7 +305,6 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
                         for (int e = 0; e < 4; e++) v[e] &= gq ? ~keep0 : keep0;
                         wg[t] = __builtin_bit_cast(h8, v);
                     }
-                    f4 D[MT][NT];
 #pragma unroll
                     for (int m = 0; m < MT; m++)
 #pragma unroll
@@ -321,18 +321,14 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
                 }
                 continue;
             }
-            f4 D[MT][NT];
 #pragma unroll
             for (int m = 0; m < MT; m++) {
 #pragma unroll
                 for (int p = 0; p < 2; p++)
 #pragma unroll
-                    for (int t = 0; t < NT; t++) {
-                        if constexpr (WT == LK_F16)
-                            y[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][m][p], w[t], y[t][m], 0, 0, 0);
-                        else
-                            D[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][m][p], w[t], p ? D[m][t] : f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    }
+                    for (int t = 0; t < NT; t++)
+                        D[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            xf[b][m][p], w[t], p || (WT == LK_F16 && b) ? D[m][t] : f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             }
             if constexpr (WT != LK_F16) {
 #pragma unroll
@@ -342,6 +338,16 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
 #pragma unroll
                         for (int i = 0; i < 4; i++) y[t][m][i] = fmaf(d[t][b], D[m][t][i], y[t][m][i]);
             }
+        }
+        // F16 has no scales, but a stage's sums of their own keep the error of an unsplit deep
+        // K down (1536 columns: 3.4e-7 with one running product, 1.3e-7 so)
+        if constexpr (WT == LK_F16) {
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) y[t][m][i] += D[m][t][i];
         }
         // the sums stay where they are: sunk to a later block by the
         // compiler, every product would be held until then
