@@ -1305,6 +1305,21 @@ static hipError_t rows_gemm(Rows& R, LkGemmArgs a, int mode, hipStream_t st) {
     return lk_gemm_launch(a, mode, st);
 }
 
+// x += the pending partials, then the RMSNorm that the GEMMs of `ws` read: as planes when
+// the tile kernel takes them all (returned true; they set planes_ready), else as xn.
+static hipError_t rows_norm(Rows& R, const float* part, uint32_t ks, uint32_t n, uint32_t h, const float* w, float eps,
+                            std::initializer_list<const LkDevW*> ws, uint32_t N, int mode, bool& planes,
+                            hipStream_t st) {
+    planes = lk_accnorm_planes_ok(h);
+    bool sums = false;
+    for (const LkDevW* q : ws) {
+        planes = planes && lk_gemm_plan(q->type, N ? N : q->rows, h, n, mode).tile.kind;
+        sums = sums || lk_planes_sums(q->type);
+    }
+    if (planes) return lk_rows_accnorm_planes_launch(R.x.as<float>(), part, ks, n, h, w, eps, sums, R.planes.p, st);
+    return lk_rows_accnorm_launch(R.x.as<float>(), part, ks, n, h, w, eps, R.xn.as<float>(), st);
+}
+
 // One pass over n rows whose meta is already on the device; logits of the
 // last row (HEAD_LAST) or of every row (HEAD_ALL, n <= LK_ROWS_LOGITS).
 // The final RMSNorm (with `pend` split-K partials still to add to x) and the
@@ -1313,10 +1328,17 @@ static hipError_t enqueue_rows_head(const lkhip_engine* e, Rows& R, uint32_t n, 
                                     int head, hipStream_t st) {
     const lkhip_config& c = e->cfg;
     const uint32_t h = c.hidden_size;
-    float *x = R.x.as<float>(), *xn = R.xn.as<float>();
-    hipError_t err = lk_rows_accnorm_launch(x, part, pend, n, h, e->norm.as<float>(), c.rms_norm_eps, xn, st);
+    float* xn = R.xn.as<float>();
+    bool planes = false;
+    hipError_t err;
+    if (head == HEAD_ALL)
+        err = rows_norm(R, part, pend, n, h, e->norm.as<float>(), c.rms_norm_eps, {&e->lm_head->dw}, 0, LK_MV_STORE,
+                        planes, st);
+    else
+        err = lk_rows_accnorm_launch(R.x.as<float>(), part, pend, n, h, e->norm.as<float>(), c.rms_norm_eps, xn, st);
     if (err != hipSuccess) return err;
     LkGemmArgs a{};
+    a.planes_ready = planes;
     a.nseg = 1;
     a.seg[0] = {e->lm_head->dw, nullptr, R.logits.as<float>()};
     a.N = c.vocab_size;
@@ -1352,8 +1374,10 @@ static hipError_t enqueue_rows(const lkhip_engine* e, Rows& R, uint32_t n, const
     uint32_t pend = 0;  // down partials of the previous layer not yet added to x
     for (uint32_t L = 0; L < c.num_hidden_layers; L++) {
         const Layer& ly = e->layers[L];
-        if (L == 0) RSTEP(lk_rmsnorm_launch(x, ly.in_norm.as<float>(), n, h, c.rms_norm_eps, xn, st));
-        else RSTEP(lk_rows_accnorm_launch(x, part, pend, n, h, ly.in_norm.as<float>(), c.rms_norm_eps, xn, st));
+        const bool mixed = qkv_mixed(ly);
+        bool planes = false;
+        RSTEP(rows_norm(R, part, pend, n, h, ly.in_norm.as<float>(), c.rms_norm_eps,
+                        {&ly.q->dw, &ly.k->dw, &ly.v->dw}, mixed ? 0 : qkvd, LK_MV_STORE, planes, st));
         uint32_t ks = 0;
         {
             LkGemmArgs a{};
@@ -1369,7 +1393,8 @@ static hipError_t enqueue_rows(const lkhip_engine* e, Rows& R, uint32_t n, const
             a.ldy = qkvd;
             a.part = part;
             a.planes = R.planes.p;
-            if (!qkv_mixed(ly)) {
+            a.planes_ready = planes;
+            if (!mixed) {
                 RSTEP(lk_gemm_launch(a, LK_MV_STORE, st, &ks));
             } else {
                 // one GEMM per projection, each reduced (bias included) into
@@ -1441,9 +1466,11 @@ static hipError_t enqueue_rows(const lkhip_engine* e, Rows& R, uint32_t n, const
             a.planes = R.planes.p;
             RSTEP(lk_gemm_launch(a, LK_MV_ACC, st, &ks));
         }
-        RSTEP(lk_rows_accnorm_launch(x, part, ks, n, h, ly.post_norm.as<float>(), c.rms_norm_eps, xn, st));
+        RSTEP(rows_norm(R, part, ks, n, h, ly.post_norm.as<float>(), c.rms_norm_eps, {&ly.gate->dw, &ly.up->dw}, I,
+                        LK_MV_SWIGLU, planes, st));
         {
             LkGemmArgs a{};
+            a.planes_ready = planes;
             a.nseg = 2;
             a.seg[0] = {ly.gate->dw, nullptr, inner};
             a.seg[1] = {ly.up->dw, nullptr, nullptr};

@@ -450,6 +450,18 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
     else store(std::true_type{});
 }
 
+// One lane's 8 scaled columns (group g) to the planes, and with `xsum` their sum with
+// the neighbour's; all lanes of the wave call it (the sums cross lanes)
+__device__ __forceinline__ void store_group(const float* o, uint32_t g, uint32_t rt, uint32_t rr, uint32_t nck,
+                                            u4* xp, float* xsum) {
+    if (g < nck * 16) lk_store_planes(xp, rt, rr, nck, g, o);
+    if (xsum) {
+        float s = ((o[0] + o[1]) + (o[2] + o[3])) + ((o[4] + o[5]) + (o[6] + o[7]));
+        s += __shfl_xor(s, 1, 64);
+        if (g % 2 == 0 && g < nck * 16) xsum[((size_t)rt * nck * 8 + g / 2) * 16 + rr] = s;
+    }
+}
+
 // Four activation rows per block, WPR waves each (rows past the last, up to a
 // whole 16-row tile, are zero): the row's power-of-two scale, its f16 planes
 // in MFMA order [row tile][chunk][block][plane][lane], the scale that undoes
@@ -508,12 +520,7 @@ __global__ __launch_bounds__(256 * WPR) void x_planes_kernel(const float* __rest
     auto store = [&](float* o, uint32_t g) {
 #pragma unroll
         for (int e = 0; e < 8; e++) o[e] *= inv;
-        if (g < nck * 16) lk_store_planes(xp, rt, rr, nck, g, o);
-        if (xsum) {
-            float s = ((o[0] + o[1]) + (o[2] + o[3])) + ((o[4] + o[5]) + (o[6] + o[7]));
-            s += __shfl_xor(s, 1, 64);
-            if (g % 2 == 0 && g < nck * 16) xsum[((size_t)rt * nck * 8 + g / 2) * 16 + rr] = s;
-        }
+        store_group(o, g, rt, rr, nck, xp, xsum);
     };
     if constexpr (G != 0) {
 #pragma unroll
@@ -524,6 +531,78 @@ __global__ __launch_bounds__(256 * WPR) void x_planes_kernel(const float* __rest
             store(v[0], g0 + t);
         }
     }
+}
+
+// rows_accnorm_kernel's work -- x += the split-K partials, then RMSNorm -- with
+// the normalised row written as planes only, RPB rows per block, WPR waves per
+// row, a lane holding its 8 columns throughout.  The float row that
+// x_planes_kernel would read back is never stored.
+template <int RPB, int WPR>
+__global__ __launch_bounds__(64 * RPB * WPR) void rows_accnorm_planes_kernel(
+    float* __restrict__ x, const float* __restrict__ part, uint32_t ks, uint32_t n_rows, uint32_t K,
+    const float* __restrict__ w, float eps, u4* __restrict__ xp, float* __restrict__ xsc, float* __restrict__ xsum) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row = wave / WPR;
+    const uint32_t r = blockIdx.x * RPB + row, nck = (K + 127) / 128;
+    const uint32_t g = (wave % WPR) * 64 + (threadIdx.x & 63), k = 8 * g < K ? 8 * g : 0;  // K is a multiple of 32
+    const bool in = r < n_rows && 8 * g < K;
+    __shared__ float red[2][RPB][WPR];
+    const size_t at = (size_t)(r < n_rows ? r : 0) * K + k;
+    f4 v[2], wt[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        v[c] = *lk_g((const f4*)(x + at + 4 * c));
+        wt[c] = *lk_g((const f4*)(w + k + 4 * c));
+    }
+    if (ks) {  // in split order, as gemm_reduce_kernel would, eight splits' loads in flight
+        const size_t stride = (size_t)n_rows * K;
+        f4 a[2] = {};
+        for (uint32_t z0 = 0; z0 < ks; z0 += 8) {
+            f4 p[8][2];
+#pragma unroll
+            for (uint32_t z = 0; z < 8; z++)
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+                    p[z][c] = *lk_g((const f4*)(part + at + (size_t)(z0 + z < ks ? z0 + z : z0) * stride + 4 * c));
+#pragma unroll
+            for (uint32_t z = 0; z < 8; z++)
+                if (z0 + z < ks) a[0] += p[z][0], a[1] += p[z][1];
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            v[c] += a[c];
+            if (in) *(f4*)(x + at + 4 * c) = v[c];
+        }
+    }
+    auto across = [&](float u, float* rd, auto op) {  // the row's WPR waves
+        if constexpr (WPR > 1) {
+            if ((threadIdx.x & 63) == 0) rd[wave % WPR] = u;
+            __syncthreads();
+            u = rd[0];
+#pragma unroll
+            for (int i = 1; i < WPR; i++) u = op(u, rd[i]);
+        }
+        return u;
+    };
+    float o[8], ss = 0.f, mx = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        o[e] = in ? v[e / 4][e % 4] : 0.f;
+        ss = fmaf(o[e], o[e], ss);
+    }
+    ss = across(lk_wave_sum(ss), red[0][row], [](float a, float b) { return a + b; });
+    const float scale = 1.0f / sqrtf(ss / (float)K + eps);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        o[e] = in ? __fmul_rn(__fmul_rn(o[e], scale), wt[e / 4][e % 4]) : 0.f;
+        mx = fmaxf(mx, fabsf(o[e]));
+    }
+    mx = across(lk_wave_max(mx), red[1][row], [](float a, float b) { return fmaxf(a, b); });
+    float inv, sc;
+    lk_row_scale(mx, inv, sc);
+    if (g == 0) xsc[r] = sc;
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[e] *= inv;
+    store_group(o, g, r / 16, r % 16, nck, xp, xsum);
 }
 
 template <int WT, int NW, int NT, int MT, bool SW, uint32_t RING, int KG = 1>
@@ -574,6 +653,24 @@ hipError_t lk_planes_launch(const float* x, uint32_t ldx, uint32_t n_rows, uint3
     else if (groups <= 768) LK_XP(4, 3);
     else LK_XP(4, 0);
 #undef LK_XP
+    return hipGetLastError();
+}
+
+hipError_t lk_rows_accnorm_planes_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
+                                         const float* w, float eps, bool sums, void* planes, hipStream_t st) {
+    if (rows == 0) return hipSuccess;
+    if (!lk_accnorm_planes_ok(n)) return hipErrorInvalidValue;
+    const LkPlanes p = lk_planes_at(planes, rows, n);
+    const uint32_t groups = (n + 127) / 128 * 16, up = (rows + 15) / 16 * 16;
+    float* const xsum = sums ? p.xsum : nullptr;
+#define LK_NP(rpb, wpr)                                                                                     \
+    hipLaunchKernelGGL((lkt::rows_accnorm_planes_kernel<rpb, wpr>), dim3(up / rpb), dim3(64 * rpb * wpr), 0, st, x, \
+                       part, ks, rows, n, w, eps, (lkt::u4*)p.xp, p.xsc, xsum)
+    if (groups <= 64) LK_NP(4, 1);
+    else if (groups <= 128) LK_NP(4, 2);
+    else if (groups <= 256) LK_NP(2, 4);
+    else LK_NP(2, 8);
+#undef LK_NP
     return hipGetLastError();
 }
 

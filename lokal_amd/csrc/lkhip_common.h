@@ -418,6 +418,11 @@ hipError_t lk_gemm_launch(LkGemmArgs a, int mode, hipStream_t st, uint32_t* defe
 //  x[r] += sum_z part[z][r] (ks > 0), then y[r] = rmsnorm(x[r]) * w
 hipError_t lk_rows_accnorm_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
                                   const float* w, float eps, float* y, hipStream_t st);
+//  the same with the normalised rows written as planes (gemm_tile.hip), for GEMMs that all take the
+//  tile kernel; a row fits one block's lanes
+inline bool lk_accnorm_planes_ok(uint32_t n) { return n % 32 == 0 && n <= 4096; }
+hipError_t lk_rows_accnorm_planes_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
+                                         const float* w, float eps, bool sums, void* planes, hipStream_t st);
 //  qkv[r] = sum_z part[z][r] + bias (ks > 0), then the rope_kv work of
 //  lk_rope_kv_launch (rotated q back into qkv, k/v into the cache)
 hipError_t lk_rows_rope_kv_launch(float* qkv, const float* part, uint32_t ks, const float* bq, const float* bk,

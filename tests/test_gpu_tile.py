@@ -8,8 +8,9 @@ import numpy as np
 import pytest
 
 import oracle
+from lokal_amd import Engine, synth
 from lokal_amd import kernels as K
-from lokal_amd import synth
+from lokal_amd.config import ModelConfig
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +74,26 @@ def test_matmul_tiles_match_float64(t, rows, cols, n):
     K.matmul(w, xd, n, y, bias=bd, accumulate=True, ldx=ldx, ldy=ldy)
     twice = y.numpy()[:, :rows]
     assert np.max(np.abs(twice - (2 * want + bias)) / (2 * scale + np.abs(bias) + 1e-300)) < bar
+
+
+@pytest.mark.parametrize("h,heads,kv,n,t,v", [
+    (256, 4, 4, 273, synth.Q8_0, None),          # one wave per row in the norm that writes the operand planes
+    (448, 7, 1, 353, synth.F16, None),           # a row that ends inside a 128-column chunk
+    (1024, 16, 8, 401, synth.Q4_K, synth.Q6_K),  # q / k / v of two types read the same planes
+    (2048, 32, 4, 100, synth.Q8_0, None),
+    (4096, 64, 8, 65, synth.Q4_K, None),         # the widest the engine takes of most types
+])
+def test_prompt_through_planes_matches_oracle(h, heads, kv, n, t, v):
+    """A prompt, and every position's logits of its first 65, of a two-layer
+    model, ragged row tiles included; within the model tests' 1e-3."""
+    cfg = ModelConfig(h, 512, 2, heads, kv, 4096, 1e-5, 1e4)
+    tensors = synth.synth_model(cfg, t, 5, tied=True, type_of=lambda _, p: v if v and p == "v_proj" else t)
+    eng, om = Engine.from_tensors(cfg, tensors), oracle.Model(cfg, tensors)
+    toks = np.random.default_rng(h).integers(0, cfg.vocab_size, n).astype(np.uint32)
+    s, s2, o = eng.session(n, kv_dtype="f32"), eng.session(n, kv_dtype="f32"), om.session(n)
+    want = [o.forward(int(x), i) for i, x in enumerate(toks)]
+    got = list(s.forward_batch(toks[:65], 0)) + [s2.prefill(toks)]
+    for g, w in zip(got, want[:65] + want[-1:]):
+        assert np.max(np.abs(g - w)) < 1e-3 * np.max(np.abs(w))
+    for x in (s, s2, o, eng, om):
+        x.close()
