@@ -731,11 +731,13 @@ static hipError_t launch_wide_k(const LkGemmArgs& a, hipStream_t st) {
     }
     return hipErrorNotSupported;
 }
-static bool wide_k_ok(uint32_t type, uint32_t K) {
-    const char* g = getenv("LKHIP_GEMM_WIDE");  // "0": gemm16_kernel for these shapes too
-    if (g && strcmp(g, "0") == 0) return false;
+static bool wide_k_fits(uint32_t type, uint32_t K) {
     const uint32_t nck = (K + KC - 1) / KC;
     return nck >= 4 && (type == LK_Q8_0 ? nck <= 7 : (type == LK_F16 ? nck <= 5 : false));
+}
+static bool wide_k_ok(uint32_t type, uint32_t K) {
+    const char* g = getenv("LKHIP_GEMM_WIDE");  // "0": gemm16_kernel for these shapes too
+    return !(g && strcmp(g, "0") == 0) && wide_k_fits(type, K);
 }
 
 // Sums the K-split partials of element (b, n) in split order, then the epilogue.
@@ -804,7 +806,8 @@ static uint32_t gemm_mb(uint32_t n_rows) { return n_rows <= 16 ? 1 : 2; }
 #define LK_GEMM_WIDE_N 16384u
 #endif
 
-// gemm_tile.hip from 33 rows on, where the product is large enough to pay for
+// gemm_tile.hip from 17 rows on (its tiles are 32 rows high; 16 rows of 32000 x 2048 Q4_K
+// take 24.5 us on gemm16_kernel, 25 there), where the product is large enough to pay for
 // its X conversion launch (2.5-8 us): from 200,000 sums.  Both sides measured
 // (us on the device, the kernels that read X themselves / the tile kernels,
 // conversion and K-split sums included): Q8_0 4864 x 896 at 64 / 512 rows
@@ -812,7 +815,7 @@ static uint32_t gemm_mb(uint32_t n_rows) { return n_rows <= 16 ? 1 : 2; }
 // 48.6 / 32.8, 1152 x 896 at 64 rows 9.3 / 10.7, 4035 x 4032 at 50 rows 28.9 /
 // 24.9, 151936 x 896 at 64 rows 105.5 / 53.2; F16 576 x 1536 at 256 rows 13.7
 // / 17.1, 1536 x 576 15.0 / 10.1; Q4_K 2048 x 5632 at 256 rows 78.7 / 38.9.
-#define LK_TILE_MIN_ROWS 33u
+#define LK_TILE_MIN_ROWS 17u
 #define LK_TILE_MIN_SUMS 200000u
 static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_rows, int mode) {
     LkTilePlan p{};
@@ -841,7 +844,16 @@ static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_ro
     //   Q8_0 151936 x 896, 64 rows: 72 / - / 55 / 110 (large 47).
     const uint32_t small = blocks(64, 32);
     uint32_t ks = 1;
-    if (sw) {
+    if (n_rows <= 32) {
+        // One row of 32-row tiles, never split over the grid: gemm16_kernel's split partials
+        // and their sum cost more than the idle CUs.  gemm16_kernel / small / deep, with the
+        // planes' own launch (3-5 us, none where the norm writes them): Q4_K 32000 x 2048, 24 rows
+        // 44.2 / 30.4 / 35.1; 11264 x 2048 28.1 / 22.1 / 20.4; Q8_0 9728 x 896 14.8 / 11.8 / 11.0;
+        // Q8_SM 32000 x 2048 52.6 / 35.5; F16 12288 x 576, 17 rows 12.6 / 9.7.  The lm_heads of
+        // gemm16_wide_kernel stay there (151936 x 896, 17 rows: 47.1 / 48.6).
+        if (!sw && N >= LK_GEMM_WIDE_N && lkg::wide_k_fits(type, K)) return p;
+        p.kind = small > 256 || (!sw && type == LK_F16) ? LK_TILE_SMALL : LK_TILE_DEEP;
+    } else if (sw) {
         p.kind = blocks(64, 64) >= 256 ? LK_TILE_LARGE : LK_TILE_SMALL;
         if (p.kind == LK_TILE_SMALL) ks = 192 / small;
     } else if (blocks(128, 64) >= 1024) {

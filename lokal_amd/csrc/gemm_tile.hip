@@ -619,6 +619,7 @@ static hipError_t launch_t(const LkGemmArgs& a, int mode, uint32_t kind, hipStre
     constexpr bool ONE = WT == LK_F16;  // no wave groups
     if (mode == LK_MV_SWIGLU) {
         if (kind == LK_TILE_SMALL) return launch<WT, 4, 2, 2, true, 2, ONE ? 1 : 2>(a, mode, st);
+        if (kind == LK_TILE_DEEP) return launch<WT, 2, 2, 2, true, 2, 4>(a, mode, st);
         return launch<WT, 4, 2, 4, true, 2>(a, mode, st);
     }
     switch (kind) {

@@ -389,7 +389,7 @@ enum LkTileKind : uint32_t {
     LK_TILE_MID = 2,    // 64 x 64, 2 stages (SwiGLU: as LK_TILE_LARGE; not Q8_SM)
     LK_TILE_LARGE = 3,  // 128 x 64 (SwiGLU: 64 x 64), 2 stages
     LK_TILE_SPLIT = 4,  // 256 x 64 by 8 waves, 2 stages
-    LK_TILE_DEEP = 5    // 64 x 32, four wave groups of 2 stages (not SwiGLU, not F16)
+    LK_TILE_DEEP = 5    // 64 x 32 (SwiGLU: 32 x 32), four wave groups of 2 stages (F16: SwiGLU only)
 };
 struct LkTilePlan {
     uint32_t kind;

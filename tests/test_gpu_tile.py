@@ -39,6 +39,11 @@ CASES = [  # type, output rows, columns, activation rows
     (synth.Q8_0, 905, 192, 250),      # four wave groups for three stages
     (synth.Q4_K, 1041, 1792, 380),    # four wave groups, a deep K
     (synth.F16, 1041, 1504, 380),     # one group, a deep K
+    (synth.Q8_0, 11771, 960, 17),     # one row of tiles: the fewest rows
+    (synth.Q8_0, 16401, 1088, 32),
+    (synth.Q4_K, 32001, 256, 24),
+    (synth.Q6_K, 11265, 768, 31),
+    (synth.F16, 12293, 608, 18),
 ]
 
 
@@ -76,17 +81,22 @@ def test_matmul_tiles_match_float64(t, rows, cols, n):
     assert np.max(np.abs(twice - (2 * want + bias)) / (2 * scale + np.abs(bias) + 1e-300)) < bar
 
 
-@pytest.mark.parametrize("h,heads,kv,n,t,v", [
-    (256, 4, 4, 273, synth.Q8_0, None),          # one wave per row in the norm that writes the operand planes
-    (448, 7, 1, 353, synth.F16, None),           # a row that ends inside a 128-column chunk
-    (1024, 16, 8, 401, synth.Q4_K, synth.Q6_K),  # q / k / v of two types read the same planes
-    (2048, 32, 4, 100, synth.Q8_0, None),
-    (4096, 64, 8, 65, synth.Q4_K, None),         # the widest the engine takes of most types
+@pytest.mark.parametrize("h,heads,kv,inter,n,t,v", [
+    (256, 4, 4, 512, 273, synth.Q8_0, None),          # one wave per row in the norm that writes the operand planes
+    (448, 7, 1, 512, 353, synth.F16, None),           # a row that ends inside a 128-column chunk
+    (1024, 16, 8, 512, 401, synth.Q4_K, synth.Q6_K),  # q / k / v of two types read the same planes
+    (2048, 32, 4, 512, 100, synth.Q8_0, None),
+    (4096, 64, 8, 512, 65, synth.Q4_K, None),         # the widest the engine takes of most types
+    (1024, 16, 2, 4864, 24, synth.Q8_0, None),        # gate / up of few rows, 32 x 32 tiles
+    (256, 4, 4, 4096, 31, synth.Q4_K, None),
+    (448, 7, 1, 4000, 30, synth.F16, None),
+    (512, 8, 2, 4352, 25, synth.Q6_K, None),
+    (256, 4, 2, 16640, 17, synth.Q8_0, None),         # more of them than CUs
 ])
-def test_prompt_through_planes_matches_oracle(h, heads, kv, n, t, v):
+def test_prompt_through_planes_matches_oracle(h, heads, kv, inter, n, t, v):
     """A prompt, and every position's logits of its first 65, of a two-layer
     model, ragged row tiles included; within the model tests' 1e-3."""
-    cfg = ModelConfig(h, 512, 2, heads, kv, 4096, 1e-5, 1e4)
+    cfg = ModelConfig(h, inter, 2, heads, kv, 4096, 1e-5, 1e4)
     tensors = synth.synth_model(cfg, t, 5, tied=True, type_of=lambda _, p: v if v and p == "v_proj" else t)
     eng, om = Engine.from_tensors(cfg, tensors), oracle.Model(cfg, tensors)
     toks = np.random.default_rng(h).integers(0, cfg.vocab_size, n).astype(np.uint32)
