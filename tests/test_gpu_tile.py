@@ -86,7 +86,7 @@ def test_matmul_tiles_match_float64(t, rows, cols, n):
     (448, 7, 1, 512, 353, synth.F16, None),           # a row that ends inside a 128-column chunk
     (1024, 16, 8, 512, 401, synth.Q4_K, synth.Q6_K),  # q / k / v of two types read the same planes
     (2048, 32, 4, 512, 100, synth.Q8_0, None),
-    (4096, 64, 8, 512, 65, synth.Q4_K, None),         # the widest the engine takes of most types
+    (4096, 64, 8, 512, 65, synth.Q4_K, None),         # the widest model the engine takes
     (1024, 16, 2, 4864, 24, synth.Q8_0, None),        # gate / up of few rows, 32 x 32 tiles
     (256, 4, 4, 4096, 31, synth.Q4_K, None),
     (448, 7, 1, 4000, 30, synth.F16, None),
