@@ -393,7 +393,8 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
     // its partial sums, else the bias, residual or SwiGLU epilogue runs here
     // (src/model.rs:27-35, :235-237, :247-249).
     const bool part = a.ks > 1;
-    const uint32_t np = part ? (SW ? 2 * a.N : a.N) : a.ldy, r0 = rt0 * 16;
+    const size_t np = part ? (SW ? 2 * (size_t)a.N : a.N) : a.ldy;
+    const uint32_t r0 = rt0 * 16;
     f4 s4[MT];
 #pragma unroll
     for (int m = 0; m < MT; m++) {
@@ -413,10 +414,10 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
                 if (a.nseg > 1 && on[t] >= e0) sg = &a.seg[1], nb = e0;
                 if (a.nseg > 2 && on[t] >= e1) sg = &a.seg[2], nb = e1;
             }
-            // uniform base: the block's first row; this lane's offset: its row and output
+            // this lane's first row and output; the other rows are uniform steps of np from it, in 64
+            // bits: 63 rows of 68.2 million floats (ldy is the caller's) pass 2^32
             float* const base = (part ? a.part + (size_t)blockIdx.z * a.n_rows * np + on[t] : sg->out + (on[t] - nb)) +
-                                (size_t)r0 * np;
-            const uint32_t o = 4 * j * np + c16;
+                                (size_t)(r0 + 4 * j) * np + c16;
             if (on[t] + c16 >= a.N) continue;
             const float bias = !part && sg->bias ? sg->bias[on[t] - nb + c16] : 0.f;
             float old[MT][4];
@@ -425,14 +426,14 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
                 for (int m = 0; m < MT; m++)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        old[m][i] = !GUARD || r0 + 16 * m + 4 * j + i < a.n_rows ? *lk_g(base + (o + (16 * m + i) * np)) : 0.f;
+                        old[m][i] = !GUARD || r0 + 16 * m + 4 * j + i < a.n_rows ? *lk_g(base + (16 * m + i) * np) : 0.f;
             }
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     if (GUARD && r0 + 16 * m + 4 * j + i >= a.n_rows) continue;
-                    float* const ob = base + (o + (16 * m + i) * np);
+                    float* const ob = base + (16 * m + i) * np;
                     float v = y[t][m][i] * s4[m][i];
                     if constexpr (SW) {
                         const float u = y[t + NO][m][i] * s4[m][i];

@@ -10,6 +10,7 @@ import pytest
 import oracle
 from lokal_amd import Engine, synth
 from lokal_amd import kernels as K
+from lokal_amd._lib import check, lib
 from lokal_amd.config import ModelConfig
 
 pytestmark = pytest.mark.gpu
@@ -79,6 +80,29 @@ def test_matmul_tiles_match_float64(t, rows, cols, n):
     K.matmul(w, xd, n, y, bias=bd, accumulate=True, ldx=ldx, ldy=ldy)
     twice = y.numpy()[:, :rows]
     assert np.max(np.abs(twice - (2 * want + bias)) / (2 * scale + np.abs(bias) + 1e-300)) < bar
+
+
+@pytest.mark.parametrize("rows,n,ldy", [
+    (32741, 64, 68_300_001),   # 64-row tiles: row 63 starts past 2^32 floats
+    (6301, 32, 138_700_003),   # 32-row tiles: row 31 does
+])
+def test_matmul_output_rows_past_2_pow_32_floats(rows, n, ldy):
+    """An output row stride at which the rows of one tile lie more than 2^32
+    floats apart: every row is stored, and accumulated, in its own place."""
+    cols = 64
+    data = synth.gen_weight(synth.Q8_0, 11, f"w{rows}x{cols}", rows, cols).data
+    w = K.Weight(synth.Q8_0, rows, cols, data)
+    x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    xd, y, small = K.DeviceArray.from_numpy(x), K.DeviceArray(((n - 1) * ldy + rows,)), K.DeviceArray((n, rows))
+    K.matmul(w, xd, n, small)
+    K.matmul(w, xd, n, y, ldy=ldy)
+    K.matmul(w, xd, n, y, accumulate=True, ldy=ldy)
+    want = small.numpy()
+    got = np.empty(rows, np.float32)
+    for r in range(n):
+        check(lib().lkhip_memcpy_dtoh(got.ctypes.data, y.ptr.value + 4 * r * ldy, got.nbytes))
+        assert np.array_equal(got, 2 * want[r]), r
+    y.free()
 
 
 @pytest.mark.parametrize("h,heads,kv,inter,n,t,v", [
