@@ -21,6 +21,7 @@
 #include "fused.h"
 #include "batch_step.h"
 #include "gguf.h"
+#include "matmul_ws.h"
 #include "repack.h"
 
 // ------------------------------------------------------------------ errors
@@ -189,85 +190,19 @@ static int weight_create(uint32_t type, size_t rows, size_t cols, const void* ho
     return LKHIP_OK;
 }
 
-// lkhip_matmul's workspaces (X planes, split-K partials), kept per stream: calls
-// on one stream run in order, so they share one buffer, and a call holds the
-// lock until its launches are enqueued, so another thread's cannot come between.
-// hipMallocAsync + hipFreeAsync cost 13 us per call, more than a small product.
-// Kept only for streams whose end is seen: the null stream and those of
-// lkhip_stream_create; other streams (and a stream that is being captured,
-// whose graph may replay beside later calls) allocate in stream order.  At most
-// kWsMost buffers of kWsBytes each; all are freed with the last weight handle.
-struct MatmulWs {
-    int device;
-    hipStream_t stream;
-    void* p;
-    size_t bytes;
-};
-static constexpr size_t kWsBytes = (size_t)256 << 20, kWsMost = 16;
-static std::mutex g_ws_mu;
-static std::vector<MatmulWs> g_ws;
-static std::vector<std::pair<int, hipStream_t>> g_own_streams;  // made by lkhip_stream_create, by device
-static size_t g_ws_weights = 0;                                  // live weight handles
-
-// The kept buffer of (current device, st) with room for `bytes`, or null; g_ws_mu is held.
-static void* ws_get(hipStream_t st, size_t bytes) {
-    int dev = 0;
-    if (bytes > kWsBytes || hipGetDevice(&dev) != hipSuccess) return nullptr;
-    if (st) {
-        if (std::find(g_own_streams.begin(), g_own_streams.end(), std::make_pair(dev, st)) == g_own_streams.end())
-            return nullptr;
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
-    }
-    for (MatmulWs& w : g_ws)
-        if (w.device == dev && w.stream == st) {
-            if (w.bytes >= bytes) return w.p;
-            void* p = nullptr;
-            const size_t want = std::max(bytes, std::min(kWsBytes, 2 * w.bytes));
-            if (hipMallocAsync(&p, want, st) != hipSuccess) return nullptr;
-            (void)hipFreeAsync(w.p, st);  // after the calls that use it
-            w.p = p;
-            w.bytes = want;
-            return p;
-        }
-    if (g_ws.size() >= kWsMost) return nullptr;
-    void* p = nullptr;
-    const size_t want = std::max<size_t>(bytes, (size_t)4 << 20);
-    if (hipMallocAsync(&p, want, st) != hipSuccess) return nullptr;
-    g_ws.push_back({dev, st, p, want});
-    return p;
-}
-// Frees the buffers of one stream (device, st), or of all; g_ws_mu is held.
-static void ws_drop(bool all, int device, hipStream_t st) {
-    for (size_t i = 0; i < g_ws.size();)
-        if (all || (g_ws[i].device == device && g_ws[i].stream == st)) {
-            (void)hipFree(g_ws[i].p);  // waits for the device
-            g_ws[i] = g_ws.back();
-            g_ws.pop_back();
-        } else {
-            i++;
-        }
-}
-static void ws_weight_created() {
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    g_ws_weights++;
-}
-static void ws_weight_destroyed() {
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    if (--g_ws_weights == 0) ws_drop(true, 0, nullptr);
-}
+static lkws::Pool g_ws;  // lkhip_matmul's workspaces
 
 extern "C" int lkhip_weight_create(uint32_t type, size_t rows, size_t cols, const void* host, size_t nbytes,
                                    lkhip_weight** out) {
     if (type == LKHIP_F32) return fail(LKHIP_E_UNSUPPORTED, "F32 matrices are not a matvec weight type here");
     const int rc = weight_create(type, rows, cols, host, nbytes, 0, out);
-    if (rc == LKHIP_OK) ws_weight_created();
+    if (rc == LKHIP_OK) lkws::weight_created(g_ws);
     return rc;
 }
 extern "C" void lkhip_weight_destroy(lkhip_weight* w) {
     if (!w) return;
     delete w;
-    ws_weight_destroyed();
+    lkws::weight_destroyed(g_ws);
 }
 extern "C" double lkhip_weight_bytes(const lkhip_weight* w) { return w ? w->bytes : 0.0; }
 
@@ -2333,24 +2268,11 @@ extern "C" int lkhip_synchronize(void) {
 extern "C" int lkhip_stream_create(void** s) {
     if (!s) return fail(LKHIP_E_INVALID, "null argument");
     HIP_OR_FAIL(hipStreamCreateWithFlags((hipStream_t*)s, hipStreamNonBlocking));
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        std::lock_guard<std::mutex> lk(g_ws_mu);
-        g_own_streams.emplace_back(dev, *(hipStream_t*)s);
-    }
+    lkws::stream_created(g_ws, *(hipStream_t*)s);
     return LKHIP_OK;
 }
 extern "C" int lkhip_stream_destroy(void* s) {
-    {
-        std::lock_guard<std::mutex> lk(g_ws_mu);
-        for (size_t i = 0; i < g_own_streams.size();)
-            if (g_own_streams[i].second == (hipStream_t)s) {
-                ws_drop(false, g_own_streams[i].first, (hipStream_t)s);
-                g_own_streams.erase(g_own_streams.begin() + i);
-            } else {
-                i++;
-            }
-    }
+    lkws::stream_destroyed(g_ws, (hipStream_t)s);
     HIP_OR_FAIL(hipStreamDestroy((hipStream_t)s));
     return LKHIP_OK;
 }
@@ -2426,17 +2348,23 @@ extern "C" int lkhip_matmul(const lkhip_weight* w, const float* x, size_t n_rows
     if (ldx < d.cols || ldy < d.rows || ldx % 4 || (uintptr_t)x % 16)
         return fail(LKHIP_E_INVALID, "matmul: ldx must be >= cols and a multiple of 4, x 16-byte aligned, ldy >= rows");
     const int mode = accumulate ? LK_MV_ACC : LK_MV_STORE;
-    const LkGemmPlan p = lk_gemm_plan(d.type, d.rows, d.cols, (uint32_t)n_rows, mode);
+    LkGemmPlan p = lk_gemm_plan(d.type, d.rows, d.cols, (uint32_t)n_rows, mode);
     hipStream_t st = (hipStream_t)stream;
-    const size_t part_bytes = (p.part_floats * 4 + 255) / 256 * 256, bytes = part_bytes + p.plane_bytes;
-    std::unique_lock<std::mutex> lk(g_ws_mu, std::defer_lock);
-    if (bytes) lk.lock();
-    void* const kept = bytes ? ws_get(st, bytes) : nullptr;
-    void* part = kept;
-    if (bytes && !kept) {
-        lk.unlock();
-        HIP_OR_FAIL(hipMallocAsync(&part, bytes, st));
+    auto part_bytes = [&] {
+        const uint32_t ks = p.tile.kind ? p.tile.ks : p.ks;
+        return ks > 1 ? (ks * n_rows * d.rows * 4 + 255) / 256 * 256 : 0;
+    };
+    lkws::Scratch ws(g_ws, st);
+    size_t bytes = part_bytes() + p.plane_bytes;
+    void* part = bytes ? ws.get(bytes) : nullptr;
+    if (bytes && !part && p.tile.kind) {
+        // no memory for the planes: the kernels that read X itself, which need less or none
+        p.tile.kind = 0;
+        p.plane_bytes = 0;
+        bytes = part_bytes();
+        part = bytes ? ws.get(bytes) : nullptr;
     }
+    if (bytes && !part) return fail(LKHIP_E_HIP, "matmul: no device memory for a workspace of %zu bytes", bytes);
     LkGemmArgs a{};
     a.nseg = 1;
     a.seg[0] = {d, bias, y};
@@ -2446,11 +2374,10 @@ extern "C" int lkhip_matmul(const lkhip_weight* w, const float* x, size_t n_rows
     a.x = x;
     a.ldx = (uint32_t)ldx;
     a.ldy = (uint32_t)ldy;
-    a.part = p.part_floats ? (float*)part : nullptr;
-    a.planes = p.plane_bytes ? (uint8_t*)part + part_bytes : nullptr;
+    a.part = (float*)part;
+    a.planes = p.plane_bytes ? (uint8_t*)part + part_bytes() : nullptr;
     a.ks = p.tile.kind ? p.tile.ks : p.ks;
     hipError_t e = lk_gemm_launch(a, mode, st);
-    if (bytes && !kept) (void)hipFreeAsync(part, st);
     if (e != hipSuccess) return fail(LKHIP_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     return LKHIP_OK;
 }

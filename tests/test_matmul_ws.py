@@ -1,0 +1,127 @@
+"""lkhip_matmul's workspaces (lokal_amd/csrc/matmul_ws.h) on the CPU, over a
+stand-in for the few HIP calls they make: a device of a given size that refuses
+what does not fit, and keeps the last error until it is read, as HIP does."""
+import ctypes as C
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+HIP = r"""
+#pragma once
+#include <cstddef>
+enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2 };
+typedef struct FakeStream* hipStream_t;
+enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0, hipStreamCaptureStatusActive = 1 };
+hipError_t hipGetDevice(int* d);
+hipError_t hipSetDevice(int d);
+hipError_t hipGetLastError();
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st);
+hipError_t hipMallocAsync(void** p, size_t n, hipStream_t s);
+hipError_t hipFreeAsync(void* p, hipStream_t s);
+hipError_t hipFree(void* p);
+"""
+PROBE = r"""
+#include <map>
+#include <mutex>
+#include <cstdint>
+#include "matmul_ws.h"
+static std::mutex mu;
+static std::map<void*, size_t> live;
+static size_t room_left, device_waits;
+static hipError_t last;
+static uintptr_t next_ptr = 4096;
+static hipStream_t capturing;
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError() { std::lock_guard<std::mutex> l(mu); const hipError_t e = last; last = hipSuccess; return e; }
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
+    *st = s && s == capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) {
+    std::lock_guard<std::mutex> l(mu);
+    if (n > room_left) return last = hipErrorOutOfMemory;
+    room_left -= n;
+    *p = (void*)(next_ptr += 4096);
+    live[*p] = n;
+    return hipSuccess;
+}
+hipError_t hipFreeAsync(void* p, hipStream_t) {
+    std::lock_guard<std::mutex> l(mu);
+    room_left += live.at(p);
+    live.erase(p);
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) { device_waits++; return hipFreeAsync(p, nullptr); }
+
+static lkws::Pool* pool;
+extern "C" {
+void start(size_t bytes) { delete pool; pool = new lkws::Pool; live.clear(); room_left = bytes; last = hipSuccess; capturing = nullptr; device_waits = 0; }
+// one call with a workspace of n bytes: whether it had one, and the bytes allocated while it ran
+int call(hipStream_t s, size_t n, size_t* held) {
+    lkws::Scratch ws(*pool, s);
+    void* p = ws.get(n);
+    size_t sum = 0;
+    for (auto& kv : live) sum += kv.second;
+    *held = sum;
+    return p != nullptr;
+}
+int last_error() { return (int)hipGetLastError(); }
+size_t held() { size_t sum = 0; for (auto& kv : live) sum += kv.second; return sum; }
+void made(hipStream_t s) { lkws::stream_created(*pool, s); }
+void ended(hipStream_t s) { lkws::stream_destroyed(*pool, s); }
+void weight(int made) { made ? lkws::weight_created(*pool) : lkws::weight_destroyed(*pool); }
+}
+"""
+MB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def ws(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("g++ not available")
+    d = tmp_path_factory.mktemp("ws")
+    (d / "hip").mkdir()
+    (d / "hip" / "hip_runtime_api.h").write_text(HIP)
+    (d / "probe.cpp").write_text(PROBE)
+    subprocess.run([gxx, "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-pthread", "-I", str(d), "-I",
+                    str(ROOT / "lokal_amd" / "csrc"), str(d / "probe.cpp"), "-o", str(d / "probe.so")], check=True)
+    lib = C.CDLL(str(d / "probe.so"))
+    lib.start.argtypes = [C.c_size_t]
+    lib.call.argtypes = [C.c_void_p, C.c_size_t, C.c_void_p]
+    lib.held.restype = C.c_size_t
+    lib.made.argtypes = lib.ended.argtypes = [C.c_void_p]
+
+    def call(stream, n):
+        held = C.c_size_t()
+        return lib.call(stream, n, C.byref(held)), held.value
+
+    lib.run = call
+    return lib
+
+
+def test_growth_that_does_not_fit(ws):
+    """A kept buffer asks for twice its size to grow; where that does not fit, the
+    call still gets what it needs, and no error is left for the launch checks."""
+    ws.start(10 * MB)
+    assert ws.run(None, 3 * MB) == (1, 4 * MB)
+    assert ws.run(None, 5 * MB)[0] == 1  # 8 MB beside the 4 do not fit
+    assert ws.last_error() == 0 and ws.held() == 5 * MB
+    assert ws.run(None, 10 * MB)[0] == 1  # nor 10 beside the 5
+    assert ws.last_error() == 0 and ws.held() == 10 * MB
+
+
+@pytest.mark.parametrize("stream", [None, 1, 2])
+def test_no_memory_leaves_no_error(ws, stream):
+    """A workspace larger than the device, on a kept stream (None, 1) or another."""
+    ws.start(6 * MB)
+    ws.made(1)
+    assert ws.run(stream, MB)[0] == 1
+    assert ws.run(stream, 7 * MB)[0] == 0
+    assert ws.last_error() == 0
+    assert ws.run(stream, 6 * MB)[0] == 1  # nothing is held on to
+    assert ws.last_error() == 0
