@@ -233,7 +233,9 @@ int lkhip_memcpy_dtoh(void* dst, const void* src, size_t bytes);
 int lkhip_memcpy_dtod(void* dst, const void* src, size_t bytes);
 int lkhip_memset(void* dptr, int value, size_t bytes);
 int lkhip_synchronize(void);
-/* Streams at default priority and events for timing kernel-level calls. */
+/* Streams at default priority and events for timing kernel-level calls.  A
+ * stream made here may keep a workspace of lkhip_matmul: end it with
+ * lkhip_stream_destroy, which gives that back in stream order (no wait). */
 int lkhip_stream_create(void** stream);
 int lkhip_stream_destroy(void* stream);
 int lkhip_stream_synchronize(void* stream);
@@ -272,7 +274,13 @@ int lkhip_q4_k_matvec(const lkhip_weight* w, const float* x, const float* bias, 
  * batched path; lokal's Metal backend runs this as matmul_pg,
  * src/gpu/kernels.metal:1749-1985): y[r*ldy + o] = dot(W[o,:], x[r*ldx ..])
  * (+ bias[o]), or += with accumulate.  fp32 accumulation on the matrix cores.
- * Needs cols % 32 == 0 (Q4_K: % 256), ldx % 4 == 0 and a 16-byte aligned x. */
+ * Needs cols % 32 == 0 (Q4_K: % 256), ldx % 4 == 0 and a 16-byte aligned x.
+ * Larger products need device memory besides (partial sums, converted x).  On
+ * the null stream and on streams of lkhip_stream_create it is kept between
+ * calls, one buffer per stream, up to 64 MiB each and 16 of them, until the
+ * stream is destroyed or the last weight is; calls on one stream from several
+ * threads take turns.  Other streams, streams being captured and larger
+ * buffers allocate and free in stream order. */
 int lkhip_matmul(const lkhip_weight* w, const float* x, size_t n_rows, size_t ldx, const float* bias, float* y,
                  size_t ldy, int accumulate, void* stream);
 /* math::rmsnorm (src/math.rs:45-49) over n_rows rows of n: y = x*s*w. */

@@ -1,35 +1,40 @@
 // matmul_ws.h -- lkhip_matmul's workspaces (X planes, split-K partials), kept
 // per stream: calls on one stream run in order, so they share one buffer, and a
-// call holds the lock until its launches are enqueued, so another thread's cannot
-// come between.  hipMallocAsync + hipFreeAsync cost 13 us per call, more than a
-// small product takes.  Kept only for streams whose end is seen: the null stream
-// and those of lkhip_stream_create; other streams (and a stream that is being
-// captured, whose graph may replay beside later calls) allocate in stream order.
-// At most kMost buffers of kBytes each; all are freed with the last weight handle.
-// Host code only.
+// call holds that stream's lock until its launches are enqueued, so another
+// thread's cannot come between; calls on other streams are not held up.
+// hipMallocAsync + hipFreeAsync cost 13 us per call, more than a small product
+// takes.  Kept only for streams whose end is seen: the null stream and those of
+// lkhip_stream_create; other streams (and a stream that is being captured,
+// whose graph may replay beside later calls) allocate in stream order.  At most
+// kMost buffers of kBytes each (a call that needs more takes longer than its
+// allocation); a stream's is freed, in its order, when it is destroyed, and all
+// with the last weight handle.  Host code only.
 #pragma once
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <vector>
 
 namespace lkws {
 
-constexpr size_t kBytes = (size_t)256 << 20, kMost = 16;
+constexpr size_t kBytes = (size_t)64 << 20, kMost = 16;
 
 struct Kept {
-    int device;
-    hipStream_t stream;
-    void* p;
-    size_t bytes;
+    int device = 0;
+    hipStream_t stream = nullptr;
+    std::mutex mu;  // the rest
+    void* p = nullptr;
+    size_t bytes = 0;
+    bool ended = false;
 };
 
 struct Pool {
     Pool() { kept.reserve(kMost); }  // nothing below throws through the C entry points
-    std::mutex mu;
-    std::vector<Kept> kept;
+    std::mutex mu;                   // never taken with a Kept's held
+    std::vector<std::shared_ptr<Kept>> kept;
     std::vector<std::pair<int, hipStream_t>> streams;  // made by lkhip_stream_create, by device
     size_t weights = 0;                                // live weight handles
 };
@@ -42,52 +47,58 @@ inline void* alloc(size_t bytes, hipStream_t st) {
     return nullptr;
 }
 
-// The kept buffer of (current device, st) with room for `bytes`, or null; pool.mu is held.
-// It asks for more than the call needs so that it grows seldom, and, where that much is
-// not to be had, for the call's own size, the old buffer given back first.
-inline void* room(Pool& pool, hipStream_t st, size_t bytes) {
+// The entry of (current device, st), or null where none is kept.
+inline std::shared_ptr<Kept> find(Pool& pool, hipStream_t st) {
     int dev = 0;
-    if (bytes > kBytes || hipGetDevice(&dev) != hipSuccess) return nullptr;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    std::lock_guard<std::mutex> lk(pool.mu);
     if (st) {
         if (std::find(pool.streams.begin(), pool.streams.end(), std::make_pair(dev, st)) == pool.streams.end())
             return nullptr;
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
     }
-    for (size_t i = 0; i < pool.kept.size(); i++) {
-        Kept& w = pool.kept[i];
-        if (w.device != dev || w.stream != st) continue;
-        if (w.bytes >= bytes) return w.p;
-        size_t want = std::max(bytes, std::min(kBytes, 2 * w.bytes));
-        void* p = alloc(want, st);
-        (void)hipFreeAsync(w.p, st);  // after the calls that use it
-        if (!p) p = alloc(want = bytes, st);
-        if (!p) {
-            pool.kept.erase(pool.kept.begin() + i);
-            return nullptr;
-        }
-        w.p = p;
-        w.bytes = want;
-        return p;
-    }
+    for (const auto& k : pool.kept)
+        if (k->device == dev && k->stream == st) return k;
     if (pool.kept.size() >= kMost) return nullptr;
-    size_t want = std::max<size_t>(bytes, (size_t)4 << 20);
-    void* p = alloc(want, st);
-    if (!p) p = alloc(want = bytes, st);
-    if (p) pool.kept.push_back({dev, st, p, want});
+    try {
+        auto k = std::make_shared<Kept>();
+        k->device = dev;
+        k->stream = st;
+        pool.kept.push_back(k);
+        return k;
+    } catch (const std::bad_alloc&) {
+        return nullptr;
+    }
+}
+
+// The entry's buffer with room for `bytes`, or null; its lock is held.  It asks for
+// more than the call needs so that it grows seldom, and, where that much is not to
+// be had, for the call's own size, the old buffer given back first.
+inline void* room(Kept& k, size_t bytes) {
+    if (k.ended || k.bytes >= bytes) return k.ended ? nullptr : k.p;
+    size_t want = std::max(bytes, std::min(kBytes, std::max((size_t)4 << 20, 2 * k.bytes)));
+    void* p = alloc(want, k.stream);
+    if (k.p) (void)hipFreeAsync(k.p, k.stream);  // after the calls that use it
+    if (!p) p = alloc(want = bytes, k.stream);
+    k.p = p;
+    k.bytes = p ? want : 0;
     return p;
 }
 
-// Frees the buffers of one stream (device, st), or of all; pool.mu is held.
-inline void drop(Pool& pool, bool all, int device, hipStream_t st) {
-    for (size_t i = 0; i < pool.kept.size();)
-        if (all || (pool.kept[i].device == device && pool.kept[i].stream == st)) {
-            (void)hipFree(pool.kept[i].p);  // waits for the device
-            pool.kept[i] = pool.kept.back();
-            pool.kept.pop_back();
-        } else {
-            i++;
-        }
+// Gives the entry's buffer back after the calls on its stream that use it; other
+// streams are not waited for, nor a capture on one of them disturbed.
+inline void end(Kept& k) {
+    std::lock_guard<std::mutex> lk(k.mu);
+    k.ended = true;
+    if (!k.p) return;
+    int dev = 0;
+    const bool other = hipGetDevice(&dev) == hipSuccess && dev != k.device;
+    if (other) (void)hipSetDevice(k.device);
+    (void)hipFreeAsync(k.p, k.stream);
+    if (other) (void)hipSetDevice(dev);
+    k.p = nullptr;
+    k.bytes = 0;
 }
 
 inline void weight_created(Pool& pool) {
@@ -95,8 +106,16 @@ inline void weight_created(Pool& pool) {
     pool.weights++;
 }
 inline void weight_destroyed(Pool& pool) {
+    std::vector<std::shared_ptr<Kept>> gone;
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        if (--pool.weights) return;
+        gone.swap(pool.kept);
+    }
+    for (const auto& k : gone) end(*k);
+    gone.clear();
     std::lock_guard<std::mutex> lk(pool.mu);
-    if (--pool.weights == 0) drop(pool, true, 0, nullptr);
+    if (pool.kept.empty()) pool.kept.swap(gone);  // its capacity
 }
 inline void stream_created(Pool& pool, hipStream_t st) {
     int dev = 0;
@@ -107,15 +126,22 @@ inline void stream_created(Pool& pool, hipStream_t st) {
     } catch (const std::bad_alloc&) {  // as a stream that was made elsewhere
     }
 }
+// Before the stream is destroyed.
 inline void stream_destroyed(Pool& pool, hipStream_t st) {
-    std::lock_guard<std::mutex> lk(pool.mu);
-    for (size_t i = 0; i < pool.streams.size();)
-        if (pool.streams[i].second == st) {
-            drop(pool, false, pool.streams[i].first, st);
-            pool.streams.erase(pool.streams.begin() + i);
-        } else {
-            i++;
-        }
+    std::shared_ptr<Kept> gone;
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        const auto s = std::find_if(pool.streams.begin(), pool.streams.end(), [&](auto& v) { return v.second == st; });
+        if (s == pool.streams.end()) return;
+        pool.streams.erase(s);
+        for (size_t i = 0; i < pool.kept.size(); i++)
+            if (pool.kept[i]->stream == st) {
+                gone = std::move(pool.kept[i]);
+                pool.kept.erase(pool.kept.begin() + i);
+                break;
+            }
+    }
+    if (gone) end(*gone);
 }
 
 // One call's workspace: the stream's kept buffer, locked, or an allocation in stream order.
@@ -124,9 +150,11 @@ public:
     Scratch(Pool& pool, hipStream_t st) : pool_(pool), st_(st) {}
     // `bytes` of device memory until this object ends, or null where there are none.
     void* get(size_t bytes) {
-        lk_ = std::unique_lock<std::mutex>(pool_.mu);
-        if (void* p = room(pool_, st_, bytes)) return p;
-        lk_.unlock();
+        if (bytes <= kBytes && (kept_ = find(pool_, st_))) {
+            lk_ = std::unique_lock<std::mutex>(kept_->mu);
+            if (void* p = room(*kept_, bytes)) return p;
+            lk_.unlock();
+        }
         return own_ = alloc(bytes, st_);
     }
     ~Scratch() {
@@ -138,7 +166,8 @@ public:
 private:
     Pool& pool_;
     hipStream_t st_;
-    std::unique_lock<std::mutex> lk_;
+    std::shared_ptr<Kept> kept_;
+    std::unique_lock<std::mutex> lk_;  // released before kept_ goes
     void* own_ = nullptr;
 };
 

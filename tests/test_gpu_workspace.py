@@ -1,5 +1,7 @@
 """lkhip_matmul's kept workspaces: products that share them equal the same
 products alone."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -38,3 +40,49 @@ def test_matmul_workspace_is_shared_in_stream_order():
             st.close()
         for w in ws:
             w.close()
+
+
+def test_matmul_workspace_from_several_threads():
+    """Two threads on streams of their own and two on the null stream, products of
+    several sizes at once: each equals the same product alone.  A fifth makes and
+    destroys streams meanwhile."""
+    rng = np.random.default_rng(6)
+    cases = []
+    for rows, cols, n in [(2048, 2048, 100), (4864, 896, 64), (1024, 4864, 200)]:
+        w = K.Weight(synth.Q8_0, rows, cols, synth.gen_weight(synth.Q8_0, 3, f"{rows}", rows, cols).data)
+        x, y = K.DeviceArray.from_numpy(rng.standard_normal((n, cols)).astype(np.float32)), K.DeviceArray((n, rows))
+        K.matmul(w, x, n, y)
+        cases.append((w, x, n, y.numpy()))
+    bad = []
+
+    def work(k, st):
+        try:
+            for rep in range(12):
+                w, x, n, want = cases[(k + rep) % len(cases)]
+                y = K.DeviceArray(want.shape)
+                K.matmul(w, x, n, y, stream=st.ptr if st else None)
+                if not np.array_equal(y.numpy(), want):
+                    bad.append((k, rep))
+        except Exception as e:  # noqa: BLE001 -- told by the main thread
+            bad.append((k, e))
+
+    def come_and_go():
+        w, x, n, want = cases[0]
+        for _ in range(6):
+            st, y = K.Stream(), K.DeviceArray(want.shape)
+            K.matmul(w, x, n, y, stream=st.ptr)
+            st.synchronize()
+            if not np.array_equal(y.numpy(), want):
+                bad.append("come_and_go")
+            st.close()
+
+    streams = [K.Stream(), K.Stream(), None, None]
+    threads = [threading.Thread(target=work, args=(k, s)) for k, s in enumerate(streams)]
+    threads.append(threading.Thread(target=come_and_go))
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    for s in streams[:2]:
+        s.close()

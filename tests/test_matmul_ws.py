@@ -24,6 +24,8 @@ hipError_t hipFreeAsync(void* p, hipStream_t s);
 hipError_t hipFree(void* p);
 """
 PROBE = r"""
+#include <chrono>
+#include <future>
 #include <map>
 #include <mutex>
 #include <cstdint>
@@ -69,6 +71,20 @@ int call(hipStream_t s, size_t n, size_t* held) {
     *held = sum;
     return p != nullptr;
 }
+// whether a call on t from another thread is through (1) or waits (0) while one on s holds its workspace
+int beside(hipStream_t s, hipStream_t t) {
+    std::future<int> f;
+    bool through;
+    {
+        lkws::Scratch ws(*pool, s);
+        ws.get(1 << 20);
+        f = std::async(std::launch::async, [t] { size_t held; return call(t, 1 << 20, &held); });
+        through = f.wait_for(std::chrono::milliseconds(s == t ? 100 : 5000)) == std::future_status::ready;
+    }
+    return f.get() && through;
+}
+size_t waits() { return device_waits; }
+void capture(hipStream_t s) { capturing = s; }
 int last_error() { return (int)hipGetLastError(); }
 size_t held() { size_t sum = 0; for (auto& kv : live) sum += kv.second; return sum; }
 void made(hipStream_t s) { lkws::stream_created(*pool, s); }
@@ -93,8 +109,9 @@ def ws(tmp_path_factory):
     lib = C.CDLL(str(d / "probe.so"))
     lib.start.argtypes = [C.c_size_t]
     lib.call.argtypes = [C.c_void_p, C.c_size_t, C.c_void_p]
-    lib.held.restype = C.c_size_t
-    lib.made.argtypes = lib.ended.argtypes = [C.c_void_p]
+    lib.held.restype = lib.waits.restype = C.c_size_t
+    lib.made.argtypes = lib.ended.argtypes = lib.capture.argtypes = [C.c_void_p]
+    lib.beside.argtypes = [C.c_void_p, C.c_void_p]
 
     def call(stream, n):
         held = C.c_size_t()
@@ -125,3 +142,39 @@ def test_no_memory_leaves_no_error(ws, stream):
     assert ws.last_error() == 0
     assert ws.run(stream, 6 * MB)[0] == 1  # nothing is held on to
     assert ws.last_error() == 0
+
+
+def test_streams_do_not_wait_for_each_other(ws):
+    """A call holds its own stream's buffer only: calls on one stream share it in
+    turn, calls on two streams go on beside each other."""
+    ws.start(100 * MB)
+    ws.made(1), ws.made(2)
+    assert ws.beside(1, 2) == 1 and ws.beside(None, 1) == 1
+    assert ws.beside(1, 1) == 0 and ws.beside(None, None) == 0
+    assert ws.held() == 3 * 4 * MB
+
+
+def test_buffers_are_bounded_and_given_back(ws):
+    """At most 16 buffers, none above 64 MB, none for a stream that was not made
+    here or is being captured; a destroyed stream's and, with the last weight,
+    all of them are freed without waiting for the device."""
+    ws.start(1 << 40)
+    ws.weight(1), ws.weight(1)
+    for s in range(1, 20):
+        ws.made(s)
+        assert ws.run(s, 64 * MB)[0] == 1
+    assert ws.held() == 16 * 64 * MB
+    assert ws.run(1, 64 * MB + 1) == (1, 17 * 64 * MB + 1) and ws.held() == 16 * 64 * MB
+    assert ws.run(99, MB) == (1, 16 * 64 * MB + MB) and ws.held() == 16 * 64 * MB
+    ws.ended(3)
+    assert ws.held() == 15 * 64 * MB
+    ws.capture(19)
+    assert ws.run(19, MB) == (1, 15 * 64 * MB + MB) and ws.held() == 15 * 64 * MB
+    ws.capture(None)
+    assert ws.run(19, MB)[0] == 1 and ws.held() == 15 * 64 * MB + 4 * MB
+    ws.weight(0)
+    assert ws.held() == 15 * 64 * MB + 4 * MB
+    ws.weight(0)
+    assert ws.held() == 0 and ws.waits() == 0
+    ws.weight(1)
+    assert ws.run(5, MB)[0] == 1 and ws.held() == 4 * MB
