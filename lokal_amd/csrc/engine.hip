@@ -2354,13 +2354,23 @@ extern "C" int lkhip_matmul(const lkhip_weight* w, const float* x, size_t n_rows
         const uint32_t ks = p.tile.kind ? p.tile.ks : p.ks;
         return ks > 1 ? (ks * n_rows * d.rows * 4 + 255) / 256 * 256 : 0;
     };
-    lkws::Scratch ws(g_ws, st);
-    size_t bytes = part_bytes() + p.plane_bytes;
-    void* part = bytes ? ws.get(bytes) : nullptr;
-    if (bytes && !part && p.tile.kind) {
-        // no memory for the planes: the kernels that read X itself, which need less or none
+    auto no_planes = [&] {  // the kernels that read X itself
         p.tile.kind = 0;
         p.plane_bytes = 0;
+    };
+    lkws::Scratch ws(g_ws, st);
+    // The planes of a product that needs no workspace otherwise would be allocated by the call where
+    // none is kept.  Under capture that puts memory nodes in the graph, which it then could not
+    // be instantiated twice with; else it costs more than the planes gain up to 750 million multiply-adds
+    // (us back to back on a caller's stream, without / with planes: Q8_0 6672 x 256, 162 rows 13.7 /
+    // 15.9; F16 5157 x 448, 321 rows 19.9 / 20.7; Q8_0 94008 x 256, 35 rows 40.2 / 22.8).
+    if (p.tile.kind && p.ks <= 1 && !ws.keeps() &&
+        ((uint64_t)d.rows * d.cols * n_rows < 750000000 || lkws::capturing(st)))
+        no_planes();
+    size_t bytes = part_bytes() + p.plane_bytes;
+    void* part = bytes ? ws.get(bytes) : nullptr;
+    if (bytes && !part && p.tile.kind) {  // no memory for the planes
+        no_planes();
         bytes = part_bytes();
         part = bytes ? ws.get(bytes) : nullptr;
     }

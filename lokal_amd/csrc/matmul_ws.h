@@ -47,17 +47,19 @@ inline void* alloc(size_t bytes, hipStream_t st) {
     return nullptr;
 }
 
+inline bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return st && (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
+}
+
 // The entry of (current device, st), or null where none is kept.
 inline std::shared_ptr<Kept> find(Pool& pool, hipStream_t st) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
     std::lock_guard<std::mutex> lk(pool.mu);
-    if (st) {
-        if (std::find(pool.streams.begin(), pool.streams.end(), std::make_pair(dev, st)) == pool.streams.end())
-            return nullptr;
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
-    }
+    if (st && (std::find(pool.streams.begin(), pool.streams.end(), std::make_pair(dev, st)) == pool.streams.end() ||
+               capturing(st)))
+        return nullptr;
     for (const auto& k : pool.kept)
         if (k->device == dev && k->stream == st) return k;
     if (pool.kept.size() >= kMost) return nullptr;
@@ -148,9 +150,14 @@ inline void stream_destroyed(Pool& pool, hipStream_t st) {
 class Scratch {
 public:
     Scratch(Pool& pool, hipStream_t st) : pool_(pool), st_(st) {}
+    // whether the stream has a kept buffer
+    bool keeps() {
+        if (!kept_) kept_ = find(pool_, st_);
+        return kept_ != nullptr;
+    }
     // `bytes` of device memory until this object ends, or null where there are none.
     void* get(size_t bytes) {
-        if (bytes <= kBytes && (kept_ = find(pool_, st_))) {
+        if (bytes <= kBytes && keeps()) {
             lk_ = std::unique_lock<std::mutex>(kept_->mu);
             if (void* p = room(*kept_, bytes)) return p;
             lk_.unlock();

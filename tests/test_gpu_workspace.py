@@ -1,10 +1,12 @@
 """lkhip_matmul's kept workspaces: products that share them equal the same
 products alone."""
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
 
+import oracle
 from lokal_amd import kernels as K
 from lokal_amd import synth
 
@@ -86,3 +88,49 @@ def test_matmul_workspace_from_several_threads():
     assert not bad
     for s in streams[:2]:
         s.close()
+
+
+@pytest.mark.parametrize("rows,cols,n,memory", [(4864, 896, 512, False), (2048, 2048, 100, True)])
+def test_matmul_under_capture(rows, cols, n, memory):
+    """A product that needs no partial sums records kernels only, so its graph can
+    be instantiated twice; one that splits K allocates inside the graph.  Replays
+    on new rows, eager products between them, equal the eager result within the
+    rounding of two f32 sums of K products, (K / 32 + 40) * 2^-24 of the |terms| each."""
+    hip = C.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(n)
+    data = synth.gen_weight(synth.Q8_0, 3, "w", rows, cols).data
+    w = K.Weight(synth.Q8_0, rows, cols, data)
+    ref = np.abs(oracle.dequant_row(synth.Q8_0, data, rows * cols).reshape(rows, cols))
+    x, y, eager = K.DeviceArray((n, cols)), K.DeviceArray((n, rows)), K.DeviceArray((n, rows))
+    x.zero()
+    st, graph, num = K.Stream(), C.c_void_p(), C.c_size_t()
+    K.matmul(w, x, n, y, stream=st.ptr)
+    st.synchronize()
+    assert hip.hipStreamBeginCapture(st.ptr, 0) == 0
+    K.matmul(w, x, n, y, stream=st.ptr)
+    assert hip.hipStreamEndCapture(st.ptr, C.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(num)) == 0
+    nodes, kind, kinds = (C.c_void_p * num.value)(), C.c_int(), []
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(num)) == 0
+    for node in nodes:
+        assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+        kinds.append(kind.value)
+    assert (set(kinds) != {0}) == memory  # 0: kernels
+    execs = [C.c_void_p() for _ in range(1 if memory else 2)]
+    for ex in execs:
+        assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    for rep in range(4):
+        xv = rng.standard_normal((n, cols)).astype(np.float32)
+        x.upload(xv)
+        K.matmul(w, x, n, eager)
+        K.synchronize()
+        y.zero()
+        K.synchronize()
+        assert hip.hipGraphLaunch(execs[rep % len(execs)], st.ptr) == 0
+        st.synchronize()
+        bar = 2 * (cols / 32 + 40) * 2.0 ** -24 * (np.abs(xv) @ ref.T)
+        assert np.all(np.abs(y.numpy() - eager.numpy()) <= bar)
+    for ex in execs:
+        assert hip.hipGraphExecDestroy(ex) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    st.close()
