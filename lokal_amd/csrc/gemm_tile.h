@@ -4,12 +4,13 @@
 #include "lkhip_common.h"
 
 // The power of two that brings a row's largest |x| (mx) into [2^14, 2^15)
-// (inv) and the one that undoes it (sc).  The exponent is kept where both
-// stay finite and normal; a row of zeros takes 2^15.
+// (inv) and the one that undoes it (sc), as long as both stay finite and normal:
+// below 2^-112 a row's largest lies lower, the smallest normal number at 2^0, where
+// the planes' grid of 2^-24 still holds its 24 bits.  A row of zeros takes 2^15.
 __device__ __forceinline__ void lk_row_scale(float mx, float& inv, float& sc) {
     int ex = 0;
     (void)frexpf(mx, &ex);  // mx = f * 2^ex, f in [0.5, 1)
-    ex = mx == 0.f ? 0 : (ex < -100 ? -100 : (ex > 128 ? 128 : ex));
+    ex = mx == 0.f ? 0 : (ex < -111 ? -111 : (ex > 128 ? 128 : ex));
     inv = ldexpf(1.0f, 15 - ex);
     sc = ldexpf(1.0f, ex - 15);
 }

@@ -4,10 +4,10 @@
 // (src/model.rs:27-35) over many tokens at once.
 //
 // Two launches.  x_planes_kernel scales each activation row by a power of
-// two (its largest |x| brought into [2^14, 2^15): exact, and elements down to
-// 2^-18 of it keep all 22 bits) and splits it once into f16 hi + lo, stored in the
-// order the matrix cores read.  gemm_tile_kernel then multiplies weight tiles
-// against those planes.  gemm16_kernel, which this replaces for large products,
+// two (its largest |x| brought into [2^14, 2^15): exact) and splits it once into
+// f16 hi + lo, stored in the order the matrix cores read: elements down to 2^-17 of
+// the row's largest are held to 2^-24 of themselves, smaller ones to 2^-40 of the
+// largest.  gemm_tile_kernel then multiplies weight tiles against those planes.  gemm16_kernel, which this replaces for large products,
 // converts the same X chunk again in every one of its N / 64 column blocks:
 // that conversion, not the MFMAs, bounded it (4864 x 896 Q8_0, 512 rows: 47.6
 // us = 94 TFLOP/s; here 20.5 us + 4.9 for the planes = 175 TFLOP/s).

@@ -82,6 +82,25 @@ def test_matmul_tiles_match_float64(t, rows, cols, n):
     assert np.max(np.abs(twice - (2 * want + bias)) / (2 * scale + np.abs(bias) + 1e-300)) < bar
 
 
+def test_matmul_smallest_normal_rows():
+    """Rows down to the smallest normal numbers keep their 24 bits in the operand
+    planes: weights of up to 2032, so that the results are normal too (a sum that
+    cancels below that rounds at 2^-150)."""
+    rows, cols, n = 6061, 64, 33
+    rng = np.random.default_rng(2)
+    q = rng.integers(-127, 128, (rows, cols // 32, 32)).astype(np.int8)
+    blocks = np.empty((rows, cols // 32, 34), np.uint8)
+    blocks[..., :2] = np.frombuffer(np.float16(16).tobytes(), np.uint8)
+    blocks[..., 2:] = q.view(np.uint8)
+    ref = 16.0 * q.reshape(rows, cols).astype(np.float64)
+    x = ((1 + rng.random((n, cols))) * rng.choice([-1, 1], (n, cols)) * 2.0 ** -rng.integers(110, 127, (n, 1)))
+    x = x.astype(np.float32)
+    w, y = K.Weight(synth.Q8_0, rows, cols, blocks.reshape(-1)), K.DeviceArray((n, rows))
+    K.matmul(w, K.DeviceArray.from_numpy(x), n, y)
+    want, scale = x.astype(np.float64) @ ref.T, np.abs(x).astype(np.float64) @ np.abs(ref).T
+    assert np.all(np.abs(y.numpy() - want) <= (cols / 32 + 40) * 2.0 ** -24 * scale + 2.0 ** -150)
+
+
 @pytest.mark.parametrize("rows,n,ldy", [
     (32741, 64, 68_300_001),   # 64-row tiles: row 63 starts past 2^32 floats
     (6301, 32, 138_700_003),   # 32-row tiles: row 31 does
