@@ -1251,7 +1251,7 @@ static hipError_t rows_norm(Rows& R, const float* part, uint32_t ks, uint32_t n,
         planes = planes && lk_gemm_plan(q->type, N ? N : q->rows, h, n, mode).tile.kind;
         sums = sums || lk_planes_sums(q->type);
     }
-    if (planes) return lk_rows_accnorm_planes_launch(R.x.as<float>(), part, ks, n, h, w, eps, sums, R.planes.p, st);
+    if (planes) return lk_rows_accnorm_planes_launch(R.x.as<float>(), part, ks, n, h, w, eps, R.xn.as<float>(), sums, R.planes.p, st);
     return lk_rows_accnorm_launch(R.x.as<float>(), part, ks, n, h, w, eps, R.xn.as<float>(), st);
 }
 

@@ -15,6 +15,24 @@ __device__ __forceinline__ void lk_row_scale(float mx, float& inv, float& sc) {
     sc = ldexpf(1.0f, ex - 15);
 }
 
+// What 8 scaled values of a lane add to their row's score (the same in every lane of
+// the wave; all of them call it).  hi + lo is off by at most max(2^-24 of the value, 2^-25), so
+// values below 2^-3 keep fewer than 22 bits.  A row where more than an eighth
+// of the values that are not zero do (score > 0; 2^17 and more below the row's largest) is
+// marked, as is one with an infinity, whose lo would be inf - inf: gemm_tile_kernel
+// multiplies marked rows with f32 operands.  A row short of that loses no more
+// than 2^-39 of its largest in an eighth of its values: less than 2^-24 of the
+// |terms| of the others, which are 2^-17 of it and more.
+__device__ __forceinline__ int lk_row_score(const float* v) {
+    int s = 0;
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        s += 8 * __builtin_popcountll(__ballot(v[e] != 0.f && fabsf(v[e]) < 0.125f)) -
+             __builtin_popcountll(__ballot(v[e] != 0.f));
+    return s;
+}
+__device__ __forceinline__ bool lk_row_marked(float mx, int score) { return score > 0 || mx == INFINITY; }
+
 // Stores 8 scaled values of row rr of row tile rt, columns 8g .. 8g+7, as f16
 // hi + lo where the MFMA operand lane that multiplies them reads them.
 __device__ __forceinline__ void lk_store_planes(void* xp, uint32_t rt, uint32_t rr, uint32_t nck, uint32_t g,

@@ -5,9 +5,10 @@
 //
 // Two launches.  x_planes_kernel scales each activation row by a power of
 // two (its largest |x| brought into [2^14, 2^15): exact) and splits it once into
-// f16 hi + lo, stored in the order the matrix cores read: elements down to 2^-17 of
-// the row's largest are held to 2^-24 of themselves, smaller ones to 2^-40 of the
-// largest.  gemm_tile_kernel then multiplies weight tiles against those planes.  gemm16_kernel, which this replaces for large products,
+// f16 hi + lo, stored in the order the matrix cores read: elements down to 2^-15 of
+// the row's largest are held to 2^-24 of themselves, smaller ones to 2^-39 of the
+// largest (a row with many of those is marked and takes f32 operands, f32_tile).
+// gemm_tile_kernel then multiplies weight tiles against those planes.  gemm16_kernel, which this replaces for large products,
 // converts the same X chunk again in every one of its N / 64 column blocks:
 // that conversion, not the MFMAs, bounded it (4864 x 896 Q8_0, 512 rows: 47.6
 // us = 94 TFLOP/s; here 20.5 us + 4.9 for the planes = 175 TFLOP/s).
@@ -75,6 +76,38 @@ __device__ __forceinline__ void dma16(const void* src, void* dst) {
 }
 __device__ __forceinline__ void dma4(const void* src, void* dst) {
     __builtin_amdgcn_global_load_lds((gptr)src, (lptr)dst, 4, 0, 0);
+}
+
+// A 16 x 16 tile of Y on f32 operands (v_mfma_f32_16x16x4_f32): activation row xr and
+// weight row r of this lane (c16), chunks c0 .. c1 of K in sums of their own.  For
+// the rows that the planes cannot hold; at an eighth of their rate and without LDS,
+// so for nothing else (Q6_K 5632 x 2048, 256 rows: 47 us a call with no row marked, 58
+// with one, 168 with all; Q8_0 4864 x 896, 512 rows: 25 / 33 / 116).  One tile at a
+// time: four that share a weight load were no faster, and their registers slowed the
+// products above (Q6_K 42.5 -> 44.4 us).
+template <int WT>
+__device__ __forceinline__ f4 f32_tile(const LkDevW& w, uint32_t r, const float* xr, uint32_t K, uint32_t c0,
+                                       uint32_t c1, uint32_t j) {
+    f4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (uint32_t c = c0; c < c1; c++) {
+        const uint32_t k = c * 128 + 32 * j, kb = k < K ? k : K - 32;  // past K: in range, times zero
+        lkg::Raw<WT> raw;
+        lkg::raw_load(raw, w, r, kb);
+        f4 x[8], acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 8; q++) x[q] = *lk_g((const f4*)(xr + kb + 4 * q));
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            float wv[8];
+            lkg::dequant8<WT>(raw, s, kb, k < K, wv);
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k < K ? x[2 * s + e / 4][e % 4] : 0.f, wv[e], acc, 0, 0, 0);
+        }
+        sum += acc;
+    }
+    return sum;
 }
 
 template <int WT, int NW, int NT, int MT, bool SW, uint32_t RING, int KG>
@@ -401,6 +434,39 @@ __global__ __launch_bounds__(64 * NW * KG, 2) void gemm_tile_kernel(const LkGemm
         const uint32_t rt = rt0 + m < RT ? rt0 + m : RT - 1;
         s4[m] = *lk_g((const f4*)(a.xsc + rt * 16 + 4 * j));
     }
+    // row tiles with marked rows, by scalar loads
+    uint32_t marked = 0;
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+        const uint32_t rt = rt0 + m < RT ? rt0 + m : RT - 1;
+        const auto mk = (const __attribute__((address_space(4))) uint64_t*)(uintptr_t)(a.xmark + (size_t)rt * 16);
+        if (mk[0] | mk[1]) marked |= 1u << m;
+    }
+    if (marked) {  // those rows again on f32 operands, whose sums need no scale
+#pragma unroll 1
+        for (uint32_t q = 0; q < NT * MT; q++) {
+            const uint32_t t = q / MT, m = q % MT;
+            if (!(marked >> m & 1)) continue;
+            const uint32_t n0 = ((blockIdx.x * NW + wave) * NO + (SW ? t % NO : t)) * 16;
+            const uint32_t rt = rt0 + m < RT ? rt0 + m : RT - 1, row = rt * 16 + c16;
+            uint32_t si = SW && t >= NO ? 1 : 0, nb = 0;
+            while (!SW && si + 1 < a.nseg && n0 >= nb + a.seg[si].w.rows) nb += a.seg[si++].w.rows;
+            const LkDevW& w = a.seg[si].w;
+            const uint32_t wr = n0 - nb + c16, mk = *lk_g((const uint32_t*)(a.xmark + rt * 16 + 4 * j));
+            const f4 v = f32_tile<WT>(w, wr < w.rows ? wr : w.rows - 1,
+                                      a.x + (size_t)(row < a.n_rows ? row : a.n_rows - 1) * a.ldx, K, s_begin / 2,
+                                      (s_end + 1) / 2, j);
+#pragma unroll
+            for (int mm = 0; mm < MT; mm++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (m != (uint32_t)mm || !(mk >> 8 * i & 1)) continue;
+                    s4[mm][i] = 1.f;
+#pragma unroll
+                    for (int tt = 0; tt < NT; tt++) y[tt][mm][i] = t == (uint32_t)tt ? v[i] : y[tt][mm][i];
+                }
+        }
+    }
     const bool acc = !SW && !part && mode == LK_MV_ACC;
     // GUARD: the block's last rows lie past n_rows
     auto store = [&](auto guard) {
@@ -466,7 +532,7 @@ __device__ __forceinline__ void store_group(const float* o, uint32_t g, uint32_t
 // Four activation rows per block, WPR waves each (rows past the last, up to a
 // whole 16-row tile, are zero): the row's power-of-two scale, its f16 planes
 // in MFMA order [row tile][chunk][block][plane][lane], the scale that undoes
-// it, and with `xsum` the row's scaled sum over every 16 columns (the Q4_K and Q8_SM
+// it, its mark (lk_row_score), and with `xsum` the row's scaled sum over every 16 columns (the Q4_K and Q8_SM
 // min terms).  A lane holds its G groups of 8 columns from the load to the
 // store (G = 0: a row too wide for that is read twice).  The four rows' 16-byte
 // pieces of a 64-byte line leave one CU together; one row per block
@@ -474,11 +540,12 @@ __device__ __forceinline__ void store_group(const float* o, uint32_t g, uint32_t
 template <int WPR, int G>
 __global__ __launch_bounds__(256 * WPR) void x_planes_kernel(const float* __restrict__ x, uint32_t ldx, uint32_t n_rows,
                                                              uint32_t K, u4* __restrict__ xp, float* __restrict__ xsc,
-                                                             float* __restrict__ xsum) {
+                                                             float* __restrict__ xsum, uint8_t* __restrict__ xmark) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = blockIdx.x * 4 + wave / WPR, nck = (K + 127) / 128, rt = r / 16, rr = r % 16;
     const uint32_t t = (wave % WPR) * 64 + (threadIdx.x & 63);  // lane of the row's 64 * WPR
     __shared__ float red[4][WPR];
+    __shared__ int cnt[4][WPR];
     const bool live = r < n_rows;
     const float* xr = x + (size_t)(live ? r : 0) * ldx;
     float v[G ? G : 1][8];
@@ -517,11 +584,12 @@ __global__ __launch_bounds__(256 * WPR) void x_planes_kernel(const float* __rest
     }
     float inv, sc;
     lk_row_scale(mx, inv, sc);
-    if (t == 0) xsc[r] = sc;
+    int score = 0;
     auto store = [&](float* o, uint32_t g) {
 #pragma unroll
         for (int e = 0; e < 8; e++) o[e] *= inv;
         store_group(o, g, rt, rr, nck, xp, xsum);
+        score += lk_row_score(o);
     };
     if constexpr (G != 0) {
 #pragma unroll
@@ -532,24 +600,36 @@ __global__ __launch_bounds__(256 * WPR) void x_planes_kernel(const float* __rest
             store(v[0], g0 + t);
         }
     }
+    if constexpr (WPR > 1) {
+        if ((threadIdx.x & 63) == 0) cnt[wave / WPR][wave % WPR] = score;
+        __syncthreads();
+        score = 0;
+#pragma unroll
+        for (int i = 0; i < WPR; i++) score += cnt[wave / WPR][i];
+    }
+    if (t == 0) {
+        xsc[r] = sc;
+        xmark[r] = lk_row_marked(mx, score);
+    }
 }
 
 // rows_accnorm_kernel's work -- x += the split-K partials, then RMSNorm -- with
 // the normalised row written as planes only, RPB rows per block, WPR waves per
 // row, a lane holding its 8 columns throughout.  The float row that
-// x_planes_kernel would read back is never stored: 512 rows of 896, 5.4 us for
+// x_planes_kernel would read back is stored (y) for marked rows only: 512 rows of 896, 5.4 us for
 // rows_accnorm_kernel + 4.5 for the planes -> 5.6 (3.3 without partials, 7-8 with
 // eight, whose 14.7 MB then bound it).  Four rows per block, as their pieces make whole
 // 64-byte lines (two: 5.9 us); wider rows two, which keeps a block to 1024 threads.
 template <int RPB, int WPR>
 __global__ __launch_bounds__(64 * RPB * WPR) void rows_accnorm_planes_kernel(
     float* __restrict__ x, const float* __restrict__ part, uint32_t ks, uint32_t n_rows, uint32_t K,
-    const float* __restrict__ w, float eps, u4* __restrict__ xp, float* __restrict__ xsc, float* __restrict__ xsum) {
+    const float* __restrict__ w, float eps, float* __restrict__ y, u4* __restrict__ xp, float* __restrict__ xsc,
+    float* __restrict__ xsum, uint8_t* __restrict__ xmark) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row = wave / WPR;
     const uint32_t r = blockIdx.x * RPB + row, nck = (K + 127) / 128;
     const uint32_t g = (wave % WPR) * 64 + (threadIdx.x & 63), k = 8 * g < K ? 8 * g : 0;  // K is a multiple of 32
     const bool in = r < n_rows && 8 * g < K;
-    __shared__ float red[2][RPB][WPR];
+    __shared__ float red[3][RPB][WPR];
     const size_t at = (size_t)(r < n_rows ? r : 0) * K + k;
     f4 v[2], wt[2];
 #pragma unroll
@@ -603,10 +683,20 @@ __global__ __launch_bounds__(64 * RPB * WPR) void rows_accnorm_planes_kernel(
     mx = across(lk_wave_max(mx), red[1][row], [](float a, float b) { return fmaxf(a, b); });
     float inv, sc;
     lk_row_scale(mx, inv, sc);
-    if (g == 0) xsc[r] = sc;
+    float p[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) o[e] *= inv;
-    store_group(o, g, r / 16, r % 16, nck, xp, xsum);
+    for (int e = 0; e < 8; e++) p[e] = o[e] * inv;
+    store_group(p, g, r / 16, r % 16, nck, xp, xsum);
+    const float score = across((float)lk_row_score(p), red[2][row], [](float a, float b) { return a + b; });
+    const bool mark = lk_row_marked(mx, (int)score);
+    if (g == 0) {
+        xsc[r] = sc;
+        xmark[r] = mark;
+    }
+    if (mark && in) {
+        *(f4*)(y + at) = f4{o[0], o[1], o[2], o[3]};
+        *(f4*)(y + at + 4) = f4{o[4], o[5], o[6], o[7]};
+    }
 }
 
 template <int WT, int NW, int NT, int MT, bool SW, uint32_t RING, int KG = 1>
@@ -650,7 +740,7 @@ hipError_t lk_planes_launch(const float* x, uint32_t ldx, uint32_t n_rows, uint3
     float* const xsum = sums ? p.xsum : nullptr;
 #define LK_XP(wpr, g)                                                                                                \
     hipLaunchKernelGGL((lkt::x_planes_kernel<wpr, g>), grid, dim3(256 * wpr), 0, st, x, ldx, n_rows, K, (lkt::u4*)p.xp, \
-                       p.xsc, xsum)
+                       p.xsc, xsum, p.mark)
     if (groups <= 64) LK_XP(1, 1);
     else if (groups <= 128) LK_XP(1, 2);
     else if (groups <= 256) LK_XP(4, 1);
@@ -662,7 +752,8 @@ hipError_t lk_planes_launch(const float* x, uint32_t ldx, uint32_t n_rows, uint3
 }
 
 hipError_t lk_rows_accnorm_planes_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
-                                         const float* w, float eps, bool sums, void* planes, hipStream_t st) {
+                                         const float* w, float eps, float* y, bool sums, void* planes,
+                                         hipStream_t st) {
     if (rows == 0) return hipSuccess;
     if (!lk_accnorm_planes_ok(n)) return hipErrorInvalidValue;
     const LkPlanes p = lk_planes_at(planes, rows, n);
@@ -670,7 +761,7 @@ hipError_t lk_rows_accnorm_planes_launch(float* x, const float* part, uint32_t k
     float* const xsum = sums ? p.xsum : nullptr;
 #define LK_NP(rpb, wpr)                                                                                     \
     hipLaunchKernelGGL((lkt::rows_accnorm_planes_kernel<rpb, wpr>), dim3(up / rpb), dim3(64 * rpb * wpr), 0, st, x, \
-                       part, ks, rows, n, w, eps, (lkt::u4*)p.xp, p.xsc, xsum)
+                       part, ks, rows, n, w, eps, y, (lkt::u4*)p.xp, p.xsc, xsum, p.mark)
     if (groups <= 64) LK_NP(4, 1);
     else if (groups <= 128) LK_NP(4, 2);
     else if (groups <= 256) LK_NP(2, 4);
@@ -684,6 +775,7 @@ hipError_t lk_tile_launch(LkGemmArgs a, int mode, const LkTilePlan& p, hipStream
     a.xp = pl.xp;
     a.xsc = pl.xsc;
     a.xsum = pl.xsum;
+    a.xmark = pl.mark;
     switch (a.seg[0].w.type) {
     case LK_Q8_0: return lkt::launch_t<LK_Q8_0>(a, mode, p.kind, st);
     case LK_F16: return lkt::launch_t<LK_F16>(a, mode, p.kind, st);

@@ -363,23 +363,27 @@ struct LkGemmArgs {
     uint32_t planes_ready;
     const void* xp;    // set by lk_tile_launch
     const float *xsc, *xsum;
+    const uint8_t* xmark;
 };
 // X as f16 planes: [row tile of 16][128-column chunk][32-column block][hi, lo][64 lanes][8 halves],
-// then each row's scale, then each row's scaled sums over 16 columns [row tile][16 columns][16 rows].
+// then each row's scale, each row's scaled sums over 16 columns [row tile][16 columns][16 rows], and a
+// byte per row: 1 where the planes cannot hold it (x is read instead).
 struct LkPlanes {
     void* xp;
     float *xsc, *xsum;
+    uint8_t* mark;
 };
 // whether a weight type's product reads the sums
 inline bool lk_planes_sums(uint32_t type) { return type == LK_Q4_K || type == LK_Q8_SM; }
 inline size_t lk_planes_bytes(size_t n_rows, size_t K) {
     const size_t rows = (n_rows + 15) / 16 * 16, kp = (K + 127) / 128 * 128;
-    return rows * kp * 4 + rows * 4 + rows * (kp / 16) * 4;
+    return rows * kp * 4 + rows * 4 + rows * (kp / 16) * 4 + rows;
 }
 inline LkPlanes lk_planes_at(void* buf, size_t n_rows, size_t K) {
     const size_t rows = (n_rows + 15) / 16 * 16, kp = (K + 127) / 128 * 128;
     float* sc = (float*)((char*)buf + rows * kp * 4);
-    return LkPlanes{buf, sc, sc + rows};
+    float* const sum = sc + rows;
+    return LkPlanes{buf, sc, sum, (uint8_t*)(sum + rows * (kp / 16))};
 }
 // gemm_tile.hip's instances: output rows x activation rows of a block (SwiGLU: output rows of each of
 // gate and up), and its 64-column stages in LDS
@@ -418,12 +422,13 @@ hipError_t lk_gemm_launch(LkGemmArgs a, int mode, hipStream_t st, uint32_t* defe
 //  x[r] += sum_z part[z][r] (ks > 0), then y[r] = rmsnorm(x[r]) * w
 hipError_t lk_rows_accnorm_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
                                   const float* w, float eps, float* y, hipStream_t st);
-//  the same with the normalised rows written as planes (gemm_tile.hip), for GEMMs that all take the
-//  tile kernel: two rows of 4096 fill one block's 1024 lanes of 8 columns, and no lm_head kernel takes
+//  the same with the normalised rows written as planes (gemm_tile.hip; y: those rows as floats that the
+//  planes cannot hold), for GEMMs that all take the tile kernel and read y as their x: two rows of 4096 fill one block's 1024 lanes of 8 columns, and no lm_head kernel takes
 //  a wider model
 inline bool lk_accnorm_planes_ok(uint32_t n) { return n % 32 == 0 && n <= 4096; }
 hipError_t lk_rows_accnorm_planes_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
-                                         const float* w, float eps, bool sums, void* planes, hipStream_t st);
+                                         const float* w, float eps, float* y, bool sums, void* planes,
+                                         hipStream_t st);
 //  qkv[r] = sum_z part[z][r] + bias (ks > 0), then the rope_kv work of
 //  lk_rope_kv_launch (rotated q back into qkv, k/v into the cache)
 hipError_t lk_rows_rope_kv_launch(float* qkv, const float* part, uint32_t ks, const float* bq, const float* bk,

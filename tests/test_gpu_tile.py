@@ -82,6 +82,86 @@ def test_matmul_tiles_match_float64(t, rows, cols, n):
     assert np.max(np.abs(twice - (2 * want + bias)) / (2 * scale + np.abs(bias) + 1e-300)) < bar
 
 
+MARKED = [  # a shape of each tile, and of a K split, per type
+    (synth.Q6_K, 6061, 256, 33), (synth.Q6_K, 131007, 256, 33), (synth.Q6_K, 1041, 2816, 257),
+    (synth.Q6_K, 11265, 768, 31), (synth.Q5_K, 32751, 256, 64), (synth.Q5_K, 1041, 2816, 257),
+    (synth.Q8_0, 1553, 960, 131), (synth.Q8_0, 32741, 64, 65), (synth.Q8_0, 700, 4864, 300),
+    (synth.F16, 3001, 608, 70), (synth.F16, 33000, 96, 67), (synth.F16, 900, 1504, 250),
+    (synth.Q4_K, 4001, 256, 50), (synth.Q4_K, 32751, 256, 64), (synth.Q4_K, 1041, 2816, 257),
+]
+
+
+@pytest.mark.parametrize("t,rows,cols,n", MARKED)
+def test_matmul_rows_beyond_the_planes(t, rows, cols, n):
+    """Rows that two f16 planes of one scale cannot hold: a large element 2^18 to
+    2^100 above the rest, which meets weights of exactly zero in some outputs, and
+    infinities.  Finite outputs are off by at most (128 + K / 128 + 2) * 2^-24 of
+    the sum of |terms| (f32 sums over a 128-column chunk, then over chunks);
+    infinities and NaN are those of the f32 products, and rows beside them keep
+    the planes' bound."""
+    data = synth.gen_weight(t, 11, f"w{rows}x{cols}", rows, cols).data.copy()
+    blk, size = synth.BLK[t]
+    raw = data.view(np.uint8).reshape(rows, cols // blk, size)
+    if t in (synth.Q4_K, synth.Q5_K):
+        raw[..., 2:4] = 0           # no mins: a quant of 0 is a weight of 0
+    big = cols - 3
+    if t == synth.F16:
+        raw[::3, big] = 0
+    if t == synth.Q8_0:
+        raw[::3, big // 32, 2 + big % 32] = 0
+    ref = oracle.dequant_row(t, data, rows * cols).reshape(rows, cols).astype(np.float64)
+    assert (ref[:, big] == 0).any()
+    rng = np.random.default_rng(rows + cols + n)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    for i, e in enumerate((18, 20, 22, 26, 30, 40, 60, 100)):
+        x[1 + i, big] = np.float32(2.0 ** e)
+    x[9, : cols // 2] *= np.float32(2.0 ** -30)
+    infs = {10: [(big, np.inf)], 11: [(1, -np.inf)], 12: [(big, np.inf), (5, np.inf)],
+            13: [(big, np.inf), (5, -np.inf)], n - 1: [(cols - 1, np.inf)]}
+    for r, at in infs.items():
+        for k, v in at:
+            x[r, k] = v
+    x[14, 7] = np.nan
+    w, y = K.Weight(t, rows, cols, data), K.DeviceArray((n, rows))
+    K.matmul(w, K.DeviceArray.from_numpy(x), n, y)
+    got = y.numpy()
+    for r, at in infs.items():
+        with np.errstate(invalid="ignore"):
+            want = sum(v * ref[:, k] for k, v in at)
+        assert np.array_equal(got[r], want.astype(np.float32), equal_nan=True), r
+    assert np.isnan(got[14]).all()
+    f = [r for r in range(n) if r not in infs and r != 14]
+    want, scale = x[f].astype(np.float64) @ ref.T, np.abs(x[f]).astype(np.float64) @ np.abs(ref).T
+    err = np.abs(got[f] - want) / (scale + 1e-300)
+    mark = [i for i, r in enumerate(f) if 1 <= r <= 9]
+    assert np.max(err[mark]) < (130 + cols / 128) * 2.0 ** -24
+    assert np.max(np.delete(err, mark, 0)) < (cols / 32 + 40) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("h,heads,kv,inter,n,t,v", [
+    (256, 4, 4, 2048, 133, synth.Q8_0, None), (1024, 16, 8, 512, 401, synth.Q4_K, synth.Q6_K),
+    (2048, 32, 4, 512, 100, synth.Q6_K, None), (448, 7, 1, 2048, 130, synth.F16, None),
+])
+def test_prompt_rows_beyond_the_planes(h, heads, kv, inter, n, t, v):
+    """Norm gains that spread every row over 2^30: the norm's planes do not hold
+    it, and the products read the floats it writes beside them.  Within the model
+    tests' 1e-3 of the oracle."""
+    cfg = ModelConfig(h, inter, 2, heads, kv, 4096, 1e-5, 1e4)
+    tensors = synth.synth_model(cfg, t, 5, tied=True, type_of=lambda _, p: v if v and p == "v_proj" else t)
+    for x in tensors:
+        if "norm" in x.name:
+            x.data.view(np.float32)[::2] *= np.float32(2.0 ** -30)
+    eng, om = Engine.from_tensors(cfg, tensors), oracle.Model(cfg, tensors)
+    toks = np.random.default_rng(h).integers(0, cfg.vocab_size, n).astype(np.uint32)
+    s, s2, o = eng.session(n, kv_dtype="f32"), eng.session(n, kv_dtype="f32"), om.session(n)
+    want = [o.forward(int(x), i) for i, x in enumerate(toks)]
+    got = list(s.forward_batch(toks[:65], 0)) + [s2.prefill(toks)]
+    for g, w in zip(got, want[:65] + want[-1:]):
+        assert np.max(np.abs(g - w)) < 1e-3 * np.max(np.abs(w))
+    for x in (s, s2, o, eng, om):
+        x.close()
+
+
 def test_matmul_smallest_normal_rows():
     """Rows down to the smallest normal numbers keep their 24 bits in the operand
     planes: weights of up to 2032, so that the results are normal too (a sum that
