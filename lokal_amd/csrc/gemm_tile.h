@@ -17,18 +17,22 @@ __device__ __forceinline__ void lk_row_scale(float mx, float& inv, float& sc) {
 
 // What 8 scaled values of a lane add to their row's score (the same in every lane of
 // the wave; all of them call it).  hi + lo is off by at most max(2^-24 of the value, 2^-25), so
-// values below 2^-3 keep fewer than 22 bits.  A row where more than an eighth
-// of the values that are not zero do (score > 0; 2^17 and more below the row's largest) is
-// marked, as is one with an infinity, whose lo would be inf - inf: gemm_tile_kernel
-// multiplies marked rows with f32 operands.  A row short of that loses no more
-// than 2^-39 of its largest in an eighth of its values: less than 2^-24 of the
-// |terms| of the others, which are 2^-17 of it and more.
+// values below 2^-3 keep fewer than 22 bits.  A row where more than seven eighths
+// of the values that are not zero are that small, 2^17 and more below its largest
+// (score > 0), is marked, as is one with an infinity, whose lo would be inf - inf:
+// gemm_tile_kernel multiplies marked rows with f32 operands.  In a row short of that
+// the small values' errors add up to at most 2^-21 of what the others do (root sum of
+// squares: sqrt(7) 2^-25.8 against 2^-3), also where the largest meet zero weights;
+// f32 operands are off by 2^-20 themselves (8e-7, Q6_K 5632 x 2048).  Fewer would not do:
+// SwiGLU rows with gates of 9 and more hold an eighth to a half of such values, which
+// add nothing, and took f32 operands at a third of the speed (Q6_K 4096 x 11008, 130
+// rows: 545 us).
 __device__ __forceinline__ int lk_row_score(const float* v) {
     int s = 0;
 #pragma unroll
     for (int e = 0; e < 8; e++)
         s += 8 * __builtin_popcountll(__ballot(v[e] != 0.f && fabsf(v[e]) < 0.125f)) -
-             __builtin_popcountll(__ballot(v[e] != 0.f));
+             7 * __builtin_popcountll(__ballot(v[e] != 0.f));
     return s;
 }
 __device__ __forceinline__ bool lk_row_marked(float mx, int score) { return score > 0 || mx == INFINITY; }
