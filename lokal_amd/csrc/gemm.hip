@@ -852,9 +852,18 @@ static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_ro
         // Q8_SM 32000 x 2048 52.6 / 35.5; F16 12288 x 576, 17 rows 12.6 / 9.7.  The lm_heads of
         // gemm16_wide_kernel stay there (151936 x 896, 17 rows: 47.1 / 48.6).
         if (!sw && N >= LK_GEMM_WIDE_N && lkg::wide_k_fits(type, K)) return p;
+        // Nor a deep K on few blocks, whose length is then all that counts, while gemm16_kernel
+        // splits it (Q8_0 6400 x 4096, 32 rows 25.4 / 31.0, 9000 x 4096 34.2 / 31.5; F16 8001 x 5440,
+        // 25 rows 31.1 / 37.9, 12000 x 5632, 17 rows 44.5 / 39.1; Q4_K 6400 x 4096, 32 rows 28.9 / 32.0, 9000 x
+        // 4096 38.2 / 32.6; Q6_K 8001 x 4864, 25 rows 38.0 / 39.3, 9000 x 4096, 32 rows 42.0 / 34.1).
+        if (!sw && K >= 2048 && small < (type == LK_F16 ? 176u : type == LK_Q4_K ? 112u : 128u)) return p;
         p.kind = small > 256 || (!sw && type == LK_F16) ? LK_TILE_SMALL : LK_TILE_DEEP;
     } else if (sw) {
-        p.kind = blocks(64, 64) >= 256 ? LK_TILE_LARGE : LK_TILE_SMALL;
+        // F16's small tile has one wave group: a serial K, which shows as long as its blocks run at
+        // once (a prompt of two layers, us small / deep / gemm16_kernel: 8192 x 2048, 64 rows 277 / 252 /
+        // 266; 3328 x 2048, 48 rows 242 / 202 / 225; 264 blocks, 5632 x 2048, 96 rows: deep 4% slower)
+        p.kind = blocks(64, 64) >= 256 ? LK_TILE_LARGE
+                 : type == LK_F16 && small <= 256 ? LK_TILE_DEEP : LK_TILE_SMALL;
         if (p.kind == LK_TILE_SMALL) ks = 192 / small;
     } else if (blocks(128, 64) >= 1024) {
         p.kind = LK_TILE_LARGE;
@@ -864,8 +873,17 @@ static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_ro
         p.kind = small > 256 || type == LK_F16 ? LK_TILE_SMALL : LK_TILE_DEEP;
         ks = 192 / small;
     } else {
+        // Splits that all run at once: one such block fills a CU, and the first of a second round
+        // doubles the time (Q6_K 833 x 2816, 352 rows: 264 blocks 39.8, 240 33.7; F16 4827 x 5312, 92
+        // rows: 266 blocks 54.4, 228 39.8).  Its planes, partials and start take 22-26 us whatever the size
+        // is, which gemm16_kernel needs at about 700 million multiply-adds, later for few outputs
+        // (of many rows) and F16 (without / with planes: Q8_0 1089 x 2240, 188 rows 19.3 / 25.6, 4100 x
+        // 2752, 53 rows 23.5 / 24.8, 2966 x 2752, 123 rows 29.9 / 26.7; Q4_K 612 x 3072, 374 rows 26.8 / 29.0;
+        // Q6_K 833 x 2816, 352 rows 30.3 / 33.7; F16 794 x 4224, 313 rows 30.1 / 32.1, 7237 x 3456, 34
+        // rows 33.2 / 28.4).
+        if ((uint64_t)N * K * n_rows < (N >= 1024 ? 700000000u : type == LK_F16 ? 1100000000u : 850000000u)) return p;
         p.kind = LK_TILE_SPLIT;
-        ks = (256 + blocks(256, 64) - 1) / blocks(256, 64);
+        ks = 256 / blocks(256, 64);
     }
     if (ks > nck) ks = nck;
     if (ks < 1) ks = 1;

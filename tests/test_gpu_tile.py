@@ -45,6 +45,10 @@ CASES = [  # type, output rows, columns, activation rows
     (synth.Q4_K, 32001, 256, 24),
     (synth.Q6_K, 11265, 768, 31),
     (synth.F16, 12293, 608, 18),
+    (synth.F16, 1100, 4000, 200),     # F16's K split over 8-wave blocks, and below its size
+    (synth.F16, 1090, 4000, 160),
+    (synth.Q8_0, 8193, 2048, 32),     # one row of tiles, a deep K: the fewest blocks, and fewer
+    (synth.Q8_0, 8100, 2048, 32),
 ]
 
 
@@ -86,7 +90,7 @@ MARKED = [  # a shape of each tile, and of a K split, per type
     (synth.Q6_K, 6061, 256, 33), (synth.Q6_K, 131007, 256, 33), (synth.Q6_K, 1041, 2816, 257),
     (synth.Q6_K, 11265, 768, 31), (synth.Q5_K, 32751, 256, 64), (synth.Q5_K, 1041, 2816, 257),
     (synth.Q8_0, 1553, 960, 131), (synth.Q8_0, 32741, 64, 65), (synth.Q8_0, 700, 4864, 300),
-    (synth.F16, 3001, 608, 70), (synth.F16, 33000, 96, 67), (synth.F16, 900, 1504, 250),
+    (synth.F16, 3001, 608, 70), (synth.F16, 33000, 96, 67), (synth.F16, 1100, 4000, 200),
     (synth.Q4_K, 4001, 256, 50), (synth.Q4_K, 32751, 256, 64), (synth.Q4_K, 1041, 2816, 257),
 ]
 
@@ -216,6 +220,9 @@ def test_matmul_output_rows_past_2_pow_32_floats(rows, n, ldy):
     (448, 7, 1, 4000, 30, synth.F16, None),
     (512, 8, 2, 4352, 25, synth.Q6_K, None),
     (256, 4, 2, 16640, 17, synth.Q8_0, None),         # more of them than CUs
+    (448, 7, 1, 4000, 40, synth.F16, None),           # F16 gate / up: four wave groups,
+    (448, 7, 1, 4000, 150, synth.F16, None),          # one with more blocks than CUs,
+    (448, 7, 1, 4000, 300, synth.F16, None),          # 64 x 64 tiles
 ])
 def test_prompt_through_planes_matches_oracle(h, heads, kv, inter, n, t, v):
     """A prompt, and every position's logits of its first 65, of a two-layer
