@@ -49,6 +49,8 @@ CASES = [  # type, output rows, columns, activation rows
     (synth.F16, 1090, 4000, 160),
     (synth.Q8_0, 8193, 2048, 32),     # one row of tiles, a deep K: the fewest blocks, and fewer
     (synth.Q8_0, 8100, 2048, 32),
+    (synth.Q8_0, 1553, 6208, 131),    # rows too wide for the conversion to hold, read twice
+    (synth.Q4_K, 1553, 6400, 131),
 ]
 
 
@@ -92,6 +94,7 @@ MARKED = [  # a shape of each tile, and of a K split, per type
     (synth.Q8_0, 1553, 960, 131), (synth.Q8_0, 32741, 64, 65), (synth.Q8_0, 700, 4864, 300),
     (synth.F16, 3001, 608, 70), (synth.F16, 33000, 96, 67), (synth.F16, 1100, 4000, 200),
     (synth.Q4_K, 4001, 256, 50), (synth.Q4_K, 32751, 256, 64), (synth.Q4_K, 1041, 2816, 257),
+    (synth.Q8_0, 1553, 6208, 131), (synth.Q4_K, 1553, 6400, 131),
 ]
 
 
@@ -223,6 +226,9 @@ def test_matmul_output_rows_past_2_pow_32_floats(rows, n, ldy):
     (448, 7, 1, 4000, 40, synth.F16, None),           # F16 gate / up: four wave groups,
     (448, 7, 1, 4000, 150, synth.F16, None),          # one with more blocks than CUs,
     (448, 7, 1, 4000, 300, synth.F16, None),          # 64 x 64 tiles
+    (512, 8, 2, 2048, 60, synth.Q6_K, None),          # Q6_K / Q5_K gate / up: two wave groups, K split over the grid,
+    (512, 8, 2, 4352, 50, synth.Q5_K, None),          # not split,
+    (512, 8, 2, 4352, 250, synth.Q6_K, None),         # 64 x 64 tiles
 ])
 def test_prompt_through_planes_matches_oracle(h, heads, kv, inter, n, t, v):
     """A prompt, and every position's logits of its first 65, of a two-layer
@@ -237,4 +243,26 @@ def test_prompt_through_planes_matches_oracle(h, heads, kv, inter, n, t, v):
     for g, w in zip(got, want[:65] + want[-1:]):
         assert np.max(np.abs(g - w)) < 1e-3 * np.max(np.abs(w))
     for x in (s, s2, o, eng, om):
+        x.close()
+
+
+@pytest.mark.parametrize("h,heads,kv,vocab,n,t", [
+    (256, 4, 4, 16385, 17, synth.Q4_K),   # the fewest rows
+    (512, 8, 2, 12001, 32, synth.Q8_0),   # below the rows of gemm16_wide_kernel
+    (448, 7, 1, 11999, 29, synth.F16),
+    (512, 8, 2, 12500, 24, synth.Q6_K),
+])
+def test_lm_head_of_few_rows_reads_the_norms_planes(h, heads, kv, vocab, n, t):
+    """A vocabulary large enough that the lm_head over 17-32 rows multiplies the
+    operand planes that the final norm writes: every position's logits within
+    the model tests' 1e-3 of the oracle."""
+    cfg = ModelConfig(h, 512, 2, heads, kv, vocab, 1e-5, 1e4)
+    tensors = synth.synth_model(cfg, t, 5, tied=True)
+    eng, om = Engine.from_tensors(cfg, tensors), oracle.Model(cfg, tensors)
+    toks = np.random.default_rng(h).integers(0, vocab, n).astype(np.uint32)
+    s, o = eng.session(n, kv_dtype="f32"), om.session(n)
+    for i, g in enumerate(s.forward_batch(toks, 0)):
+        w = o.forward(int(toks[i]), i)
+        assert np.max(np.abs(g - w)) < 1e-3 * np.max(np.abs(w)), i
+    for x in (s, o, eng, om):
         x.close()
