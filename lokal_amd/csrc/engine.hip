@@ -1240,8 +1240,8 @@ static hipError_t rows_gemm(Rows& R, LkGemmArgs a, int mode, hipStream_t st) {
     return lk_gemm_launch(a, mode, st);
 }
 
-// x += the pending partials, then the RMSNorm that the GEMMs of `ws` read: as planes when
-// the tile kernel takes them all (returned true; they set planes_ready), else as xn.
+// x += the pending partials, then the RMSNorm that the GEMMs of `ws` read: as planes when the tile
+// kernel takes them all (planes is set; xn then holds the marked rows only), else as xn.
 static hipError_t rows_norm(Rows& R, const float* part, uint32_t ks, uint32_t n, uint32_t h, const float* w, float eps,
                             std::initializer_list<const LkDevW*> ws, uint32_t N, int mode, bool& planes,
                             hipStream_t st) {
@@ -1251,7 +1251,9 @@ static hipError_t rows_norm(Rows& R, const float* part, uint32_t ks, uint32_t n,
         planes = planes && lk_gemm_plan(q->type, N ? N : q->rows, h, n, mode).tile.kind;
         sums = sums || lk_planes_sums(q->type);
     }
-    if (planes) return lk_rows_accnorm_planes_launch(R.x.as<float>(), part, ks, n, h, w, eps, R.xn.as<float>(), sums, R.planes.p, st);
+    if (planes)
+        return lk_rows_accnorm_planes_launch(R.x.as<float>(), part, ks, n, h, w, eps, R.xn.as<float>(), sums,
+                                             R.planes.p, st);
     return lk_rows_accnorm_launch(R.x.as<float>(), part, ks, n, h, w, eps, R.xn.as<float>(), st);
 }
 

@@ -850,7 +850,8 @@ static LkTilePlan tile_plan(uint32_t type, uint32_t N, uint32_t K, uint32_t n_ro
         // planes' own launch (3-5 us, none where the norm writes them): Q4_K 32000 x 2048, 24 rows
         // 44.2 / 30.4 / 35.1; 11264 x 2048 28.1 / 22.1 / 20.4; Q8_0 9728 x 896 14.8 / 11.8 / 11.0;
         // Q8_SM 32000 x 2048 52.6 / 35.5; F16 12288 x 576, 17 rows 12.6 / 9.7.  The lm_heads of
-        // gemm16_wide_kernel stay there (151936 x 896, 17 rows: 47.1 / 48.6).
+        // gemm16_wide_kernel stay there (151936 x 896, 17 rows: 47.1 / 48.6); with a bias or an
+        // accumulation, which that kernel does not take, they stay on gemm16_kernel.
         if (!sw && N >= LK_GEMM_WIDE_N && lkg::wide_k_fits(type, K)) return p;
         // Nor a deep K on few blocks, whose length is then all that counts, while gemm16_kernel
         // splits it (Q8_0 6400 x 4096, 32 rows 25.4 / 31.0, 9000 x 4096 34.2 / 31.5; F16 8001 x 5440,

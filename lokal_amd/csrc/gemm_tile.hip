@@ -8,10 +8,11 @@
 // f16 hi + lo, stored in the order the matrix cores read: elements down to 2^-15 of
 // the row's largest are held to 2^-24 of themselves, smaller ones to 2^-39 of the
 // largest (a row with many of those is marked and takes f32 operands, f32_tile).
-// gemm_tile_kernel then multiplies weight tiles against those planes.  gemm16_kernel, which this replaces for large products,
-// converts the same X chunk again in every one of its N / 64 column blocks:
-// that conversion, not the MFMAs, bounded it (4864 x 896 Q8_0, 512 rows: 47.6
-// us = 94 TFLOP/s; here 20.5 us + 4.9 for the planes = 175 TFLOP/s).
+// gemm_tile_kernel then multiplies weight tiles against those planes.
+// gemm16_kernel, which this replaces for large products, converts the same X
+// chunk again in every one of its N / 64 column blocks: that conversion, not
+// the MFMAs, bounded it (4864 x 896 Q8_0, 512 rows: 47.6 us = 94 TFLOP/s; here
+// 20.4 us + 5.0 for the planes = 176 TFLOP/s).
 //
 // gemm_tile_kernel: a block of NW waves takes 16 NT NW weight rows x 16 MT
 // activation rows over a range of K, 64 columns (a stage) at a time; KG such
@@ -21,17 +22,18 @@
 // the X planes shared by the block, and each wave's own weight rows and scales
 // in the order it reads them back.  X is the MFMA's A operand and W its B, so a
 // lane's column is one weight row and the block scale is one scalar of it.
-// What bounds it: vector instructions (per MFMA pair four FMAs with the block
-// scale; ten per 8 weights to widen them, spread over MT tiles) beside the
-// MFMAs, 1.9-2.2 GHz under that load, and with few blocks the ~1 us each
-// stage's barrier, LDS reads and products take one after another.
+// What bounds it: the chain of barrier, LDS reads, widening (ten vector
+// instructions per 8 weights, spread over MT tiles), products and scaling (four
+// FMAs per MFMA pair), which two to three waves per SIMD go through one after
+// another at 1.9-2.2 GHz.  No unit is saturated (counters, 4864 x 896 Q8_0, 512 rows:
+// vector instructions issue in 39% of the cycles, MFMAs run in 28%, LDS in 31% without
+// bank conflicts; 2048 x 5632 Q4_K, 203 rows: 43 / 30 / 21%).
 #include "gemm_impl.h"
 #include "gemm_tile.h"
 
 #include <type_traits>
 
 namespace lkt {
-
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 hh2 __attribute__((ext_vector_type(2)));

@@ -423,8 +423,8 @@ hipError_t lk_gemm_launch(LkGemmArgs a, int mode, hipStream_t st, uint32_t* defe
 hipError_t lk_rows_accnorm_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
                                   const float* w, float eps, float* y, hipStream_t st);
 //  the same with the normalised rows written as planes (gemm_tile.hip; y: those rows as floats that the
-//  planes cannot hold), for GEMMs that all take the tile kernel and read y as their x: two rows of 4096 fill one block's 1024 lanes of 8 columns, and no lm_head kernel takes
-//  a wider model
+//  planes cannot hold), for GEMMs that all take the tile kernel and read y as their x: two rows of 4096
+//  fill one block's 1024 lanes of 8 columns, and no lm_head kernel takes a wider model
 inline bool lk_accnorm_planes_ok(uint32_t n) { return n % 32 == 0 && n <= 4096; }
 hipError_t lk_rows_accnorm_planes_launch(float* x, const float* part, uint32_t ks, uint32_t rows, uint32_t n,
                                          const float* w, float eps, float* y, bool sums, void* planes,
