@@ -8,7 +8,7 @@
 // whose graph may replay beside later calls) allocate in stream order.  At most
 // kMost buffers of kBytes each (a call that needs more takes longer than its
 // allocation); a stream's is freed, in its order, when it is destroyed, and all
-// with the last weight handle.  Host code only.
+// (but those of streams being captured) with the last weight handle.  Host code only.
 #pragma once
 #include <hip/hip_runtime_api.h>
 
@@ -49,7 +49,10 @@ inline void* alloc(size_t bytes, hipStream_t st) {
 
 inline bool capturing(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return st && (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
+    if (!st) return false;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
 }
 
 // The entry of (current device, st), or null where none is kept.
@@ -89,18 +92,24 @@ inline void* room(Kept& k, size_t bytes) {
 }
 
 // Gives the entry's buffer back after the calls on its stream that use it; other
-// streams are not waited for, nor a capture on one of them disturbed.
-inline void end(Kept& k) {
+// streams are not waited for, nor a capture on one of them disturbed.  On a stream that
+// is being captured itself the free would become a node of its graph: false, and the
+// entry stays, unless the stream is to be `gone`.
+inline bool end(Kept& k, bool gone) {
     std::lock_guard<std::mutex> lk(k.mu);
+    const bool cap = capturing(k.stream);
+    if (cap && !gone) return false;
     k.ended = true;
-    if (!k.p) return;
+    if (!k.p) return true;
     int dev = 0;
     const bool other = hipGetDevice(&dev) == hipSuccess && dev != k.device;
     if (other) (void)hipSetDevice(k.device);
-    (void)hipFreeAsync(k.p, k.stream);
+    if (cap) (void)hipFree(k.p);
+    else (void)hipFreeAsync(k.p, k.stream);
     if (other) (void)hipSetDevice(dev);
     k.p = nullptr;
     k.bytes = 0;
+    return true;
 }
 
 inline void weight_created(Pool& pool) {
@@ -108,16 +117,10 @@ inline void weight_created(Pool& pool) {
     pool.weights++;
 }
 inline void weight_destroyed(Pool& pool) {
-    std::vector<std::shared_ptr<Kept>> gone;
-    {
-        std::lock_guard<std::mutex> lk(pool.mu);
-        if (--pool.weights) return;
-        gone.swap(pool.kept);
-    }
-    for (const auto& k : gone) end(*k);
-    gone.clear();
     std::lock_guard<std::mutex> lk(pool.mu);
-    if (pool.kept.empty()) pool.kept.swap(gone);  // its capacity
+    if (--pool.weights) return;
+    auto& k = pool.kept;  // keeps its capacity
+    k.erase(std::remove_if(k.begin(), k.end(), [](auto& e) { return end(*e, false); }), k.end());
 }
 inline void stream_created(Pool& pool, hipStream_t st) {
     int dev = 0;
@@ -143,7 +146,7 @@ inline void stream_destroyed(Pool& pool, hipStream_t st) {
                 break;
             }
     }
-    if (gone) end(*gone);
+    if (gone) end(*gone, true);
 }
 
 // One call's workspace: the stream's kept buffer, locked, or an allocation in stream order.

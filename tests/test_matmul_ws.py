@@ -32,10 +32,11 @@ PROBE = r"""
 #include "matmul_ws.h"
 static std::mutex mu;
 static std::map<void*, size_t> live;
-static size_t room_left, device_waits;
+static size_t room_left, device_waits, recorded;
 static hipError_t last;
 static uintptr_t next_ptr = 4096;
 static hipStream_t capturing;
+static void* graphs;  // the last allocation made under capture, freed there too
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError() { std::lock_guard<std::mutex> l(mu); const hipError_t e = last; last = hipSuccess; return e; }
@@ -43,16 +44,18 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
     *st = s && s == capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
-hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) {
+hipError_t hipMallocAsync(void** p, size_t n, hipStream_t s) {
     std::lock_guard<std::mutex> l(mu);
     if (n > room_left) return last = hipErrorOutOfMemory;
     room_left -= n;
     *p = (void*)(next_ptr += 4096);
     live[*p] = n;
+    if (s && s == capturing) graphs = *p;
     return hipSuccess;
 }
-hipError_t hipFreeAsync(void* p, hipStream_t) {
+hipError_t hipFreeAsync(void* p, hipStream_t s) {
     std::lock_guard<std::mutex> l(mu);
+    if (s && s == capturing && p != graphs) { recorded++; return hipSuccess; }  // a node of the graph
     room_left += live.at(p);
     live.erase(p);
     return hipSuccess;
@@ -61,7 +64,7 @@ hipError_t hipFree(void* p) { device_waits++; return hipFreeAsync(p, nullptr); }
 
 static lkws::Pool* pool;
 extern "C" {
-void start(size_t bytes) { delete pool; pool = new lkws::Pool; live.clear(); room_left = bytes; last = hipSuccess; capturing = nullptr; device_waits = 0; }
+void start(size_t bytes) { delete pool; pool = new lkws::Pool; live.clear(); room_left = bytes; last = hipSuccess; capturing = nullptr; device_waits = recorded = 0; }
 // one call with a workspace of n bytes: whether it had one, and the bytes allocated while it ran
 int call(hipStream_t s, size_t n, size_t* held) {
     lkws::Scratch ws(*pool, s);
@@ -84,6 +87,7 @@ int beside(hipStream_t s, hipStream_t t) {
     return f.get() && through;
 }
 size_t waits() { return device_waits; }
+size_t frees_recorded() { return recorded; }
 void capture(hipStream_t s) { capturing = s; }
 int last_error() { return (int)hipGetLastError(); }
 size_t held() { size_t sum = 0; for (auto& kv : live) sum += kv.second; return sum; }
@@ -109,7 +113,7 @@ def ws(tmp_path_factory):
     lib = C.CDLL(str(d / "probe.so"))
     lib.start.argtypes = [C.c_size_t]
     lib.call.argtypes = [C.c_void_p, C.c_size_t, C.c_void_p]
-    lib.held.restype = lib.waits.restype = C.c_size_t
+    lib.held.restype = lib.waits.restype = lib.frees_recorded.restype = C.c_size_t
     lib.made.argtypes = lib.ended.argtypes = lib.capture.argtypes = [C.c_void_p]
     lib.beside.argtypes = [C.c_void_p, C.c_void_p]
 
@@ -178,3 +182,26 @@ def test_buffers_are_bounded_and_given_back(ws):
     assert ws.held() == 0 and ws.waits() == 0
     ws.weight(1)
     assert ws.run(5, MB)[0] == 1 and ws.held() == 4 * MB
+
+
+def test_no_free_is_recorded_into_a_capture(ws):
+    """The last weight goes while a stream with a kept buffer is being captured: the
+    free would become a node of that graph, so the buffer stays and is used and freed
+    later; the other streams' go.  A destroyed stream's goes in any case."""
+    ws.start(100 * MB)
+    ws.weight(1)
+    ws.made(1), ws.made(2)
+    assert ws.run(1, MB)[0] == 1 and ws.run(2, MB)[0] == 1
+    ws.capture(1)
+    ws.weight(0)
+    assert ws.frees_recorded() == 0 and ws.held() == 4 * MB
+    ws.capture(None)
+    ws.weight(1)
+    assert ws.run(1, MB) == (1, 4 * MB)
+    ws.weight(0)
+    assert ws.held() == 0
+    ws.weight(1)
+    assert ws.run(2, MB)[0] == 1
+    ws.capture(2)
+    ws.ended(2)
+    assert ws.frees_recorded() == 0 and ws.held() == 0
